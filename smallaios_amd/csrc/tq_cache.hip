@@ -117,14 +117,16 @@ __device__ __forceinline__ float load_row_elem(const void* p, size_t i, bool bf1
 }
 
 // One butterfly stage below 64: dims l and l ^ H of each lane pair into
-// (a + b, a - b), the sum at the lower dim.
+// (a + b, a - b), the sum at the lower dim: the partner plus or minus the
+// lane's own value, the sign as an exact product (no select of two sums).
 template <int H, int E>
 __device__ __forceinline__ void butterfly_stage(float (&y)[E], int lane) {
 #pragma clang fp contract(off)
+  const float own = (lane & H) ? -1.0f : 1.0f;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const float p = lane_xor<H>(y[e], lane);
-    y[e] = (lane & H) ? p - y[e] : y[e] + p;
+    y[e] = y[e] * own + p;
   }
 }
 
@@ -252,16 +254,16 @@ __device__ __forceinline__ float wave_qjl(const uint32_t (&code)[D / 64], float 
 
 // Encodes the row x (lane l: dims l + 64 e) as position r of (kv head h,
 // sequence b), K (kind 0) or V (kind 1), and stores it: K codes row-major; V
-// codes into the position's bits of its tile, in the LDS copy `stile` of the
-// tile's words when given, else by read-modify-write of the words in memory
-// (the caller guarantees that no other wave writes that tile meanwhile);
+// codes into the position's bits of its tile, by read-modify-write of the
+// words in memory (the caller guarantees that no other wave writes that tile
+// meanwhile);
 // then the parameters (scale, zero point, QJL mean, sum of the codes) and the
 // QJL sign words. Orders its LDS use at wave level only.
 template <int D, int BITS>
 __device__ __forceinline__ void wave_store_row(const TqArgs& a, const float (&x)[D / 64],
                                                const float (&sgn)[D / 64], int lane, int h, int b,
-                                               int r, int kind, uint32_t (*stile)[2 * BITS + 1],
-                                               float* sres, uint32_t* scode) {
+                                               int r, int kind, float* sres,
+                                               uint32_t* scode) {
 #pragma clang fp contract(off)
   constexpr int E = D / 64;
   constexpr int W = D * BITS / 32;  // K code words per row
@@ -296,7 +298,7 @@ __device__ __forceinline__ void wave_store_row(const TqArgs& a, const float (&x)
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int d = lane + 64 * e;
-      uint32_t* tw = stile ? stile[d] : vt + d * TBW;
+      uint32_t* tw = vt + d * TBW;
       tw[w] = (tw[w] & ~(LEVELS << sh)) | (code[e] << sh);
       if (sh + BITS > 32) tw[w + 1] = (tw[w + 1] & ~(LEVELS >> (32 - sh))) | (code[e] >> (32 - sh));
     }
@@ -316,52 +318,243 @@ __device__ __forceinline__ void wave_store_row(const TqArgs& a, const float (&x)
   if (lane == 0) (kind ? a.par_v : a.par_k)[row] = make_float4(scale, zero, c, csum);
 }
 
-// ---- write: one wave per (sequence, kv head, K|V, 64-position tile) --------
-// The wave encodes the tile's rows of this pass in order. K rows go out
-// row-major; V codes are merged into the tile's words (read, modified in LDS,
-// written back) by the one wave that owns the tile.
-template <int D, int BITS>
-__global__ __launch_bounds__(64) void tq_write_kernel(const TqArgs a, const void* k, const void* v,
-                                                      int bf16, int s_new) {
+// ---- write: one workgroup per (sequence, kv head, K|V, 64-position tile) ----
+// L = D/32 lanes hold a row, 32 consecutive dims each, so 64/L rows of the
+// pass are encoded by a wave at once. Five butterfly stages and the packing of
+// the K codes and sign words (a lane's 32 codes are BITS whole words, its 32
+// signs one) stay in the lane; the stages of 32 and up, the minimum and the
+// maximum go over L neighbouring lanes. sum|r| keeps its dim order: the lanes
+// of a row take turns, each starting from its predecessor's sum. V codes cross
+// lanes once, through LDS, into the words of the position-packed tile (old
+// bits of positions outside the pass kept); one workgroup owns a tile.
+//
+// The work is the serial arithmetic of a row (two butterflies, D IEEE
+// divisions, the D-long sum), not memory. One row per wave at a time ran
+// those chains 64 times over per tile: a 2 x 1024-row pass (8 kv heads, D =
+// 128, 4 bits, QJL, bf16; 23 MB, 3 us at 8 TB/s) took 133 us and takes 14.1 (19
+// with an IEEE division for every code).
+template <int D>
+__device__ __forceinline__ void lane32_butterfly(float (&y)[32], int lane, float norm) {
 #pragma clang fp contract(off)
-  constexpr int E = D / 64;
+#pragma unroll
+  for (int hs = 1; hs < 32; hs <<= 1)
+#pragma unroll
+    for (int e = 0; e < 32; ++e)
+      if ((e & hs) == 0) {
+        const float a0 = y[e], a1 = y[e + hs];
+        y[e] = a0 + a1;
+        y[e + hs] = a0 - a1;
+      }
+  butterfly_stage<1>(y, lane);  // dims 32 apart: neighbouring lanes
+  if constexpr (D >= 128) butterfly_stage<2>(y, lane);
+  if constexpr (D >= 256) butterfly_stage<4>(y, lane);
+#pragma unroll
+  for (int e = 0; e < 32; ++e) y[e] *= norm;
+}
+
+// Reductions over the D/32 lanes of a row.
+template <int D, typename F>
+__device__ __forceinline__ float row_reduce(float v, int lane, F&& op) {
+  v = op(v, lane_xor<1>(v, lane));
+  if constexpr (D >= 128) v = op(v, lane_xor<2>(v, lane));
+  if constexpr (D >= 256) v = op(v, lane_xor<4>(v, lane));
+  return v;
+}
+
+template <int D, int BITS>
+__global__ __launch_bounds__(2 * D) void tq_write_kernel(const TqArgs a, const void* k,
+                                                         const void* v, int bf16, int vec,
+                                                         int s_new) {
+#pragma clang fp contract(off)
+  constexpr int L = D / 32;
   constexpr int TBW = 2 * BITS;  // V words per dim per tile
-  const int lane = threadIdx.x;
+  constexpr uint32_t LEVELS = (1u << BITS) - 1u;
+  constexpr int STRIDE = D / 4 + 1;  // dwords of a row of codes in LDS
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int j = tid % L, pr = tid / L;  // dims 32j .. 32j+31 of tile position pr
   const int kind = blockIdx.y & 1, h = blockIdx.y >> 1, b = blockIdx.z;
   const int len = a.seq_lens[b];
   const int tile = len / 64 + (int)blockIdx.x;
   const int r_lo = max(len, tile * 64), r_hi = min(len + s_new, tile * 64 + 64);
   if (r_lo >= r_hi) return;  // uniform
-  __shared__ uint32_t scode[D];
-  __shared__ float sres[D];
-  __shared__ uint32_t stile[D][TBW + 1];
-  const void* src = kind ? v : k;
-  const bool is_bf16 = bf16 != 0;
-  float sgn[E];
+  __shared__ uint32_t scode[64 * STRIDE];  // V: a byte per code, [position][dim]
+  const int r = tile * 64 + pr;
+  const bool live = r >= r_lo && r < r_hi;
+  if (__ballot(live) != 0) {
+    const void* src = kind ? v : k;
+    // a lane outside the pass encodes its first row (and stores nothing)
+    const size_t in_off = (((size_t)b * s_new + ((live ? r : r_lo) - len)) * a.heads + h) * D +
+                          32 * j;
+    float x[32];
+    if (vec) {
+      if (bf16) {
 #pragma unroll
-  for (int e = 0; e < E; ++e) sgn[e] = (float)a.signs[(size_t)h * D + lane + 64 * e];
+        for (int e = 0; e < 32; e += 8) {
+          const uint4 w = *(const uint4*)((const uint16_t*)src + in_off + e);
+          const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            x[e + 2 * i] = __uint_as_float(ws[i] << 16);
+            x[e + 2 * i + 1] = __uint_as_float(ws[i] & 0xFFFF0000u);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 32; e += 4) {
+          const float4 w = *(const float4*)((const float*)src + in_off + e);
+          x[e] = w.x, x[e + 1] = w.y, x[e + 2] = w.z, x[e + 3] = w.w;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 32; ++e) x[e] = load_row_elem(src, in_off + e, bf16 != 0);
+    }
+    uint32_t sg[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sg[i] = ((const uint32_t*)(a.signs + (size_t)h * D + 32 * j))[i];
+    auto sgn = [&](int e) { return (float)(int8_t)(sg[e >> 2] >> (8 * (e & 3))); };
+
+    // PolarQuantizer::encode, as wave_encode
+    float y[32];
+#pragma unroll
+    for (int e = 0; e < 32; ++e) y[e] = x[e] * sgn(e);
+    lane32_butterfly<D>(y, lane, a.norm);
+    float mn = y[0], mx = y[0];
+#pragma unroll
+    for (int e = 1; e < 32; ++e) {
+      mn = fminf(mn, y[e]);
+      mx = fmaxf(mx, y[e]);
+    }
+    mn = row_reduce<D>(mn, lane, [](float p, float q) { return fminf(p, q); });
+    mx = row_reduce<D>(mx, lane, [](float p, float q) { return fmaxf(p, q); });
+    if (__ballot(mn == 0.0f) != 0) {
+      // a zero minimum takes the sign of the row's first zero in dim order
+      float z = 0.0f;
+      bool has = false;
+#pragma unroll
+      for (int e = 31; e >= 0; --e)
+        if (y[e] == 0.0f) {
+          z = y[e];
+          has = true;
+        }
+      const uint64_t m = (__ballot(has) >> (lane & ~(L - 1))) & ((1ull << L) - 1ull);
+      const float first = __shfl(z, (lane & ~(L - 1)) + (m ? __builtin_ctzll(m) : 0), 64);
+      if (mn == 0.0f && m) mn = first;
+    }
+    const float range = mx - mn;
+    const float scale = range > 0.0f ? range / (float)LEVELS : 1.0f;
+    const float zero = mn;
+    uint32_t cb[8] = {};  // the lane's codes, a byte each
+    float csum = 0.0f;    // integers below 2^24: exact
+    if (__ballot(!(range < INFINITY && scale >= 1e-30f)) == 0) {
+      // Finite rows: the quotient t = (y - zero) / scale >= 0 as a product with
+      // the scale's reciprocal. That is within 2^-22 t of the rounded
+      // quotient, so away from the half-integers both round to the same code;
+      // within NEAR of one, the quotient itself decides.
+      constexpr float NEAR = (float)LEVELS / (float)(1 << 20);
+      const float rs = __builtin_amdgcn_rcpf(scale);
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const float d = y[e] - zero, t = d * rs;
+        float cf = __builtin_rintf(t);
+        if (__ballot(fabsf(__builtin_amdgcn_fractf(t) - 0.5f) <= NEAR) != 0)
+          cf = round_half_away(d / scale);
+        cf = fminf(cf, (float)LEVELS);
+        cb[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(cf, e & 3, cb[e >> 2]);
+        csum += cf;
+        y[e] = cf * scale + zero;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const uint32_t q = scale > 0.0f ? sat_u32(round_half_away((y[e] - zero) / scale)) : 0u;
+        const uint32_t code = q < LEVELS ? q : LEVELS;
+        cb[e >> 2] |= code << (8 * (e & 3));
+        csum += (float)code;
+        y[e] = (float)code * scale + zero;
+      }
+    }
+    csum = row_reduce<D>(csum, lane, [](float p, float q) { return p + q; });
+    const size_t row = ((size_t)h * a.batch_cap + b) * a.rows_cap + r;
+    if (kind) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) scode[pr * STRIDE + 8 * j + i] = cb[i];
+    } else {
+      uint32_t wd[BITS] = {};
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const uint32_t code = (cb[e >> 2] >> (8 * (e & 3))) & 0xFFu;
+        const int w = (BITS * e) >> 5, sh = (BITS * e) & 31;
+        wd[w] |= code << sh;
+        if (sh + BITS > 32) wd[w + 1] |= code >> (32 - sh);
+      }
+      uint32_t* dst = (uint32_t*)(a.codes_k + row * a.code_stride) + BITS * j;
+      if (live) {
+        if constexpr (BITS % 4 == 0) {
+#pragma unroll
+          for (int i = 0; i < BITS; i += 4)
+            *(uint4*)(dst + i) = make_uint4(wd[i], wd[i + 1], wd[i + 2], wd[i + 3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < BITS; ++i) dst[i] = wd[i];
+        }
+      }
+    }
+    // QJLResidualEncoder::encode, as wave_qjl
+    float c = 0.0f;
+    if (a.qjl) {
+      lane32_butterfly<D>(y, lane, a.norm);
+      uint32_t sb = 0u;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) {
+        const float res = x[e] - y[e] * sgn(e);
+        sb |= res >= 0.0f ? 1u << e : 0u;
+        y[e] = fabsf(res);
+      }
+      float sum = 0.0f;
+#pragma unroll
+      for (int ph = 0; ph < L; ++ph) {
+#pragma unroll
+        for (int e = 0; e < 32; ++e) sum += y[e];
+        // the next lane of the row goes on from here (row_shr:1)
+        if (ph + 1 < L)
+          sum = __int_as_float(
+              __builtin_amdgcn_mov_dpp(__float_as_int(sum), 0x111, 0xF, 0xF, false));
+      }
+      c = sum / (float)D;  // the row's last lane
+      if (live) ((kind ? a.signs_v : a.signs_k) + row * L)[j] = sb;
+    }
+    if (live && j == L - 1) (kind ? a.par_v : a.par_k)[row] = make_float4(scale, zero, c, csum);
+  }
+  if (!kind) return;  // uniform
+  __syncthreads();
+  // four dims' word w of the tile per thread
   uint32_t* vt = (uint32_t*)(a.codes_v + (((size_t)h * a.batch_cap + b) * a.tiles_cap + tile) *
                                              tq_vtile_bytes(D, BITS));
-  const int w_lo = ((r_lo - tile * 64) * BITS) >> 5;
-  const int w_hi = ((r_hi - tile * 64) * BITS - 1) >> 5;
-  if (kind) {
+  const int lo = r_lo - tile * 64, hi = r_hi - tile * 64;
+  constexpr int NP = (31 + BITS - 1) / BITS + 1;  // positions with bits in a word, at most
+  for (int it = tid; it < D / 4 * TBW; it += 2 * D) {
+    const int w = it % TBW, d4 = it / TBW;
+    const int i0 = (32 * w) / BITS;
+    uint32_t mask = 0u, wd[4] = {};
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-      for (int w = w_lo; w <= w_hi; ++w) stile[lane + 64 * e][w] = vt[(lane + 64 * e) * TBW + w];
-    wave_lds_sync();
-  }
-  for (int r = r_lo; r < r_hi; ++r) {
-    const size_t in_off = (((size_t)b * s_new + (r - len)) * a.heads + h) * D;
-    float x[E];
+    for (int n = 0; n < NP; ++n) {
+      const int i = i0 + n, sh = BITS * i - 32 * w;
+      if (sh >= 32 || i < lo || i >= hi) continue;
+      const uint32_t c4 = scode[i * STRIDE + d4];
+      mask |= sh >= 0 ? LEVELS << sh : LEVELS >> -sh;
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = load_row_elem(src, in_off + lane + 64 * e, is_bf16);
-    wave_store_row<D, BITS>(a, x, sgn, lane, h, b, r, kind, stile, sres, scode);
-  }
-  if (kind) {
-    wave_lds_sync();
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t code = (c4 >> (8 * q)) & 0xFFu;
+        wd[q] |= sh >= 0 ? code << sh : code >> -sh;
+      }
+    }
+    if (mask == 0u) continue;
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-      for (int w = w_lo; w <= w_hi; ++w) vt[(lane + 64 * e) * TBW + w] = stile[lane + 64 * e][w];
+    for (int q = 0; q < 4; ++q) {
+      uint32_t* dst = vt + (4 * d4 + q) * TBW + w;
+      *dst = mask == 0xFFFFFFFFu ? wd[q] : ((*dst & ~mask) | wd[q]);
+    }
   }
 }
 
@@ -956,8 +1149,8 @@ __global__ __launch_bounds__(64 * NW, NW >= 8 ? 2 : 1) void tq_attend_kernel(
       float sgn[D / 64];
 #pragma unroll
       for (int e = 0; e < D / 64; ++e) sgn[e] = (float)a.signs[(size_t)kvh * D + lane + 64 * e];
-      wave_store_row<D, BITS>(a, xnk, sgn, lane, kvh, b, L - 1, 0, nullptr, sres[wave], scode);
-      wave_store_row<D, BITS>(a, xnv, sgn, lane, kvh, b, L - 1, 1, nullptr, sres[wave], scode);
+      wave_store_row<D, BITS>(a, xnk, sgn, lane, kvh, b, L - 1, 0, sres[wave], scode);
+      wave_store_row<D, BITS>(a, xnv, sgn, lane, kvh, b, L - 1, 1, sres[wave], scode);
       __threadfence_block();
       tq_load_tile<D, BITS, MODE>(a, rbase, vbase, first, r1, lane, tb[0]);
     }
@@ -1286,11 +1479,15 @@ hipError_t dispatch_dbits(int d, int bits, F&& f) {
 hipError_t launch_tq_write(const TqArgs& a, const void* k, const void* v, int bf16, int batch,
                            int s_new, hipStream_t st) {
   if (batch <= 0 || s_new <= 0) return hipSuccess;
+  // 16-byte loads of a lane's 32 dims need both inputs aligned (a row is a
+  // multiple of 64 bytes); the elementwise loads serve the others
+  const int vec = (((uintptr_t)k | (uintptr_t)v) & 15u) == 0;
   // tiles a pass of s_new positions can touch, whatever the start's offset
   const dim3 grid((s_new + 126) / 64, 2 * a.heads, batch);
   return dispatch_dbits(a.head_dim, a.bits, [&](auto dd, auto bb) -> hipError_t {
     constexpr int D = decltype(dd)::value, B = decltype(bb)::value;
-    hipLaunchKernelGGL((tq_write_kernel<D, B>), grid, dim3(64), 0, st, a, k, v, bf16, s_new);
+    hipLaunchKernelGGL((tq_write_kernel<D, B>), grid, dim3(2 * D), 0, st, a, k, v, bf16, vec,
+                       s_new);
     return hipGetLastError();
   });
 }

@@ -152,6 +152,51 @@ def test_writes_across_tile_boundaries(rt, d, bits):
         c.close()
 
 
+@pytest.mark.parametrize("d,bits,bf16,shift", [(64, 3, False, 1), (64, 8, True, 0),
+                                               (128, 3, True, 1), (128, 4, False, 0),
+                                               (128, 4, True, 3), (128, 8, False, 2),
+                                               (256, 3, False, 0), (256, 4, True, 1)])
+def test_write_rows_at_tile_edges(rt, d, bits, bf16, shift):
+    """Passes of 1, 62, 1, 64, 65, 16 and 17 rows: starts and ends at, before
+    and after the 64-position tiles and the rows of a wave. The inputs start
+    `shift` elements into their buffer, so the elementwise loads of inputs
+    that are not 16-byte aligned run too, and hold rows of zeros of both
+    signs, of one value, and one-hot rows. Every row bit for bit."""
+    import torch
+    log(f"tq write edges d={d} bits={bits} bf16={bf16} shift={shift}")
+    rng = np.random.default_rng(d + 7 * bits + shift)
+    batch, heads = 2, 3
+    sizes = (1, 62, 1, 64, 65, 16, 17)
+    c = S.TqCache(rt, 1, heads, d, bits, True, batch, sum(sizes), seed=SEED)
+    try:
+        ks, vs = [], []
+        for s in sizes:
+            dev = []
+            for acc in (ks, vs):
+                x = rng.standard_normal((batch, s, heads, d)).astype(np.float32)
+                x[0, s // 2, 0] = 0.0
+                x[0, s // 2, 1] = -0.0
+                x[0, s // 2, 2] = 0.25
+                x[1, s - 1, 0] = 0.0
+                x[1, s - 1, 0, d - 1] = -3.0
+                x = x.reshape(batch, s, heads * d)
+                acc.append(host_vals(x, bf16))
+                buf = torch.empty(x.size + shift, device="cuda",
+                                  dtype=torch.bfloat16 if bf16 else torch.float32)
+                buf[shift:] = to_dev(x.ravel(), bf16)
+                dev.append(buf[shift:])
+            c.write(0, dev[0], dev[1], batch, s)
+            c.advance()
+        torch.cuda.synchronize()
+        k, v = np.concatenate(ks, axis=1), np.concatenate(vs, axis=1)
+        for b in range(batch):
+            for h in range(heads):
+                check_rows(c, 0, b, h, 0, rows_of(k, b, h, heads, d), rows_of(v, b, h, heads, d),
+                           heads, d, bits, True, SEED)
+    finally:
+        c.close()
+
+
 def test_constant_and_edge_rows(rt):
     """Constant rows (range 0: scale 1.0), zeros, large magnitudes."""
     import torch
