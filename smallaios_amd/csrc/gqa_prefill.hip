@@ -12,7 +12,8 @@
 //            permuted k-order of the PV operand; rows padded so the 16-byte
 //            LDS reads are conflict-free. One barrier per tile. int8 codes are
 //            stored exactly (|code| <= 128) and their per-token scales applied
-//            to the scores and to P; int4 codes are dequantised while staged.
+//            to the scores and to P; int4 K codes are stored exactly too, V is
+//            dequantised while staged.
 //   S^T      A = K tile (LDS), B = Q^T (registers, f16 of q * scale * log2 e);
 //            lane (row r, g) receives tokens 4g+e of each 16-token block, so
 //            the row softmax is in-lane plus two cross-group reductions and P
@@ -115,15 +116,13 @@ constexpr int kPrecLift = 12;
 
 // V fragments read ahead of the PV MFMAs that consume them
 constexpr int kVPrefetch = 6;
-constexpr int kVPrefetchInt4 = 3;  // int4 keeps its K lo tile reads and has fewer spare registers
 
-template <int D, bool KLO = false>
+template <int D>
 struct PrefillTile {
   static constexpr int KROW = D + 8;      // padded f16 row of the K tile
   static constexpr int VROW = 4 * 8 + 8;  // padded f16 (kstep, dim) row: 4 groups x 8
   // every member 16-byte aligned: fragments are read with ds_read_b128
   alignas(16) _Float16 k[64 * KROW];
-  alignas(16) _Float16 klo[KLO ? 64 * KROW : 8];  // int4: K - f16(K), hi + lo hold K to ~22 bits
   alignas(16) _Float16 v[2 * D * VROW];
   alignas(16) float sk[64];
   alignas(16) float sv[64];
@@ -149,32 +148,20 @@ struct TileStage {
 };
 
 // Page ids (pool blocks) a thread's staging loads of one 64-token tile touch:
-// chunk i of the K and V loads (c = tid + NT i) lies in local page c / D for
-// int8, and in c / (16 * D/32) (K) and c / D (V) for int4; the first 128
-// threads (int8) also load one scale of token tid & 63. They are loaded one
-// tile ahead, so the tile's code loads never wait on a page-table read.
+// chunk i of the K and V loads (c = tid + NT i) lies in local page c / D, and
+// so do the int4 parameters (all three are 4 D items a tile); the first 128
+// threads (int8) also load one scale of token tid & 63. They are loaded ahead,
+// so the tile's code loads never wait on a page-table read.
 template <int D, int NT, bool INT4>
 struct StagePages {
-  static constexpr int KN = INT4 ? 64 * (D / 32) : 64 * (D / 16);  // K chunks of a tile
-  static constexpr int VN = 4 * D;                                  // V chunks of a tile
-  static constexpr int KC = (KN + NT - 1) / NT;
-  static constexpr int VC = (VN + NT - 1) / NT;
-  int k[KC];
-  int v[VC];
+  static constexpr int N = (4 * D + NT - 1) / NT;
+  int k[N];
   int s;
 
   __device__ __forceinline__ void load(const int32_t* pt, int tile, int last_page, int tid) {
 #pragma unroll
-    for (int i = 0; i < KC; ++i) {
-      const int c = min(tid + NT * i, KN - 1);
-      const int lp = INT4 ? c / (16 * (D / 32)) : c / D;
-      k[i] = pt[min(4 * tile + lp, last_page)];
-    }
-#pragma unroll
-    for (int i = 0; i < VC; ++i) {
-      const int c = min(tid + NT * i, VN - 1);
-      v[i] = pt[min(4 * tile + c / D, last_page)];
-    }
+    for (int i = 0; i < N; ++i)
+      k[i] = pt[min(4 * tile + min(tid + NT * i, 4 * D - 1) / D, last_page)];
     s = INT4 ? 0 : pt[min(4 * tile + (tid & 63) / kPageTokens, last_page)];
   }
 };
@@ -209,7 +196,7 @@ __device__ __forceinline__ void stage_load(TileStage<D, NT>& S, const PrefillPar
     const int c = tid + NT * i;
     if (TileStage<D, NT>::VN % NT != 0 && c >= TileStage<D, NT>::VN) break;
     const int d = c % D;
-    S.vc[i] = *(const uint4*)(page_block(head, P.v[i], BB) + 16 * D + d * 16);
+    S.vc[i] = *(const uint4*)(page_block(head, P.k[i], BB) + 16 * D + d * 16);
   }
   // the first 128 threads load one scale each; tokens past the sequence end
   // are zeroed when the tile is stored (a select here would wait for the load)
@@ -278,23 +265,45 @@ __device__ __forceinline__ void stage_store(const TileStage<D, NT>& S, Tile& T, 
   }
 }
 
-// ---- int4 cache: the same LDS tile, filled with dequantised f16 values -------
-// A group's scale and zero vary along head_dim, so they cannot be applied after
-// the dot product: K and V are dequantised while staged (code * s + z in f32,
-// rounded once to f16; the binary16 parameters bound the range anyway), and
-// the softmax then uses unit token scales. Tokens past the sequence end are
-// zeroed so a stale slot can never inject a NaN into the PV product.
+// ---- int4 cache ---------------------------------------------------------------
+// K = code * s + z with (s, z) per token and group of 32 dims, and a group is
+// exactly one k step of the QK product. So the K tile holds the bare codes,
+// and a score is sum over groups of s * <code, q> (one f32 multiply-add per
+// group on the product's output) plus <z, sum of q> over the groups, which is
+// one more k step: z is binary16 as stored, the sums of q go in as hi + lo.
+// K is thus exact, in two MFMAs a k step; dequantised to an f16 pair hi + lo
+// it took three, twice the K tile, and a hundred VALU operations per thread
+// and tile for the split. The codes enter as binary16 subnormals code * 2^-24
+// (a mask per two; the MFMA multiplies subnormals exactly), the factor is in
+// the staged scale. V has its groups along the output dims, so it is
+// dequantised while staged: one fma rounded once to f16 of v * 2^-5.
+// Tokens past the sequence end get zero parameters, so a stale slot cannot
+// inject a NaN.
+// 1 x 1024 over 3000 at 32Q/8KV, D = 128, keys with outlier channels: the tile
+// loop 137 -> 120 us, the call 178 -> 143 (with the query prologue below).
+//
+// The parameters of a tile are staged one tile ahead of its codes (V's are
+// needed to store them), in a ring of three.
+template <int D>
+struct Int4Params {
+  static constexpr int NG = D / 32;
+  static constexpr int ZROW = 32 + 8;  // padded row of the zero points' k step
+  alignas(16) float sk[NG * 64];       // K scale * 2^24, [group][token]
+  alignas(16) float2 sv[NG * 64];      // V (scale, zero) * 2^-5, [group][token]
+  // [token]: the groups' K zero points twice (against the hi and the lo of the
+  // query's sums), then zeros up to 32
+  alignas(16) _Float16 z[64 * ZROW];
+};
+
+// A thread's items of one tile: 8 bytes of K codes (16 dims of a token), 8
+// of V codes (16 slots of a dim) and one (scale, zero) pair, all of them
+// consecutive in a page block.
 template <int D, int NT>
 struct TileStage4 {
-  static constexpr int NG = D / 32;
-  static constexpr int KN = 64 * NG;             // K chunks: (token, group), 16 B
-  static constexpr int VN = 4 * D;               // V chunks: (page, dim), 8 B
-  static constexpr int KC = (KN + NT - 1) / NT;  // per thread
-  static constexpr int VC = (VN + NT - 1) / NT;
-  uint4 kc[KC];
-  uint32_t kp[KC];      // (scale, zero) binary16 pair of the K chunk's group
-  uint2 vc[VC];
-  uint32_t vp[VC][16];  // (scale, zero) of each of the V chunk's 16 slots
+  static constexpr int N = (4 * D + NT - 1) / NT;
+  uint2 kc[N];
+  uint2 vc[N];
+  uint32_t par[N];
 };
 
 __device__ __forceinline__ float half_lo(uint32_t w) {
@@ -306,100 +315,227 @@ __device__ __forceinline__ float half_hi(uint32_t w) {
 
 template <int D, int NT>
 __device__ __forceinline__ void stage_load4(TileStage4<D, NT>& S, const PrefillParams& p,
-                                            const StagePages<D, NT, true>& P, int kvh, int t0,
-                                            int tid) {
+                                            const StagePages<D, NT, true>& P, int kvh, int tid) {
   constexpr size_t BB = block_bytes_int4(D);
-  constexpr int NG = D / 32;
-  static_assert(StagePages<D, NT, true>::KC == TileStage4<D, NT>::KC &&
-                StagePages<D, NT, true>::VC == TileStage4<D, NT>::VC, "chunk counts");
   const uint8_t* head = head_blocks(p, kvh, BB);
 #pragma unroll
-  for (int i = 0; i < TileStage4<D, NT>::KC; ++i) {
-    const int c = min(tid + NT * i, TileStage4<D, NT>::KN - 1);  // spare threads repeat the last
-    const int tok = c / NG;
-    const int grp = c % NG;
+  for (int i = 0; i < TileStage4<D, NT>::N; ++i) {
+    const int c = min(tid + NT * i, 4 * D - 1) % D;  // spare threads repeat the last item
     const uint8_t* blk = page_block(head, P.k[i], BB);
-    const int slot = tok & 15;
-    S.kc[i] = *(const uint4*)(blk + slot * (D / 2) + 16 * grp);
-    S.kp[i] = *(const uint32_t*)(blk + 16 * D + (slot * NG + grp) * 4);
-  }
-#pragma unroll
-  for (int i = 0; i < TileStage4<D, NT>::VC; ++i) {
-    const int c = min(tid + NT * i, TileStage4<D, NT>::VN - 1);
-    const int d = c % D;
-    const uint8_t* blk = page_block(head, P.v[i], BB);
-    S.vc[i] = *(const uint2*)(blk + 8 * D + d * 8);
-    const uint8_t* par = blk + 16 * D + 64 * NG + (d / 32) * 4;
-#pragma unroll
-    for (int sl = 0; sl < 16; ++sl) S.vp[i][sl] = *(const uint32_t*)(par + (size_t)sl * NG * 4);
+    S.kc[i] = *(const uint2*)(blk + 8 * c);
+    S.vc[i] = *(const uint2*)(blk + 8 * D + 8 * c);
   }
 }
 
 template <int D, int NT>
-__device__ __forceinline__ void stage_store4(const TileStage4<D, NT>& S, PrefillTile<D, true>& T,
-                                             int t0, int total, int tid) {
-  constexpr int KROW = PrefillTile<D, true>::KROW;
-  constexpr int VROW = PrefillTile<D, true>::VROW;
+__device__ __forceinline__ void params_load4(TileStage4<D, NT>& S, const PrefillParams& p,
+                                             const StagePages<D, NT, true>& P, int kvh, int tid) {
+  constexpr size_t BB = block_bytes_int4(D);
+  const uint8_t* head = head_blocks(p, kvh, BB);
+#pragma unroll
+  for (int i = 0; i < TileStage4<D, NT>::N; ++i) {
+    const int c = min(tid + NT * i, 4 * D - 1) % D;
+    S.par[i] = *(const uint32_t*)(page_block(head, P.k[i], BB) + 16 * D + 4 * c);
+  }
+}
+
+template <int D, int NT>
+__device__ __forceinline__ void params_store4(const TileStage4<D, NT>& S, Int4Params<D>& Z, int t0,
+                                              int total, int tid) {
   constexpr int NG = D / 32;
 #pragma unroll
-  for (int i = 0; i < TileStage4<D, NT>::KC; ++i) {
+  for (int i = 0; i < TileStage4<D, NT>::N; ++i) {
     const int c = tid + NT * i;
-    if (c >= TileStage4<D, NT>::KN) break;
-    const int tok = c / NG;
-    const int grp = c % NG;
-    const bool valid = t0 + tok < total;
-    const float sc = half_lo(S.kp[i]), zr = half_hi(S.kp[i]);
-    const uint32_t w[4] = {S.kc[i].x, S.kc[i].y, S.kc[i].z, S.kc[i].w};
-    uint32_t h[16], l[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      // elements 2j, 2j+1: nibbles 2j, 2j+1 of the chunk (LSB first); the
-      // value code * s + z (code * s exact in f32) as an f16 pair hi + lo
-      const uint32_t wj = w[j >> 2] >> (8 * (j & 3));
-      float a = valid ? (float)(wj & 0xF) * sc + zr : 0.0f;
-      float b = valid ? (float)((wj >> 4) & 0xF) * sc + zr : 0.0f;
-      // one rounded value feeds both halves of the split
-      __asm__("" : "+v"(a), "+v"(b));
-      const _Float16 ah = (_Float16)a, bh = (_Float16)b;
-      h[j] = __builtin_bit_cast(uint32_t, v2h{ah, bh});
-      l[j] = __builtin_bit_cast(uint32_t, v2h{(_Float16)(a - (float)ah), (_Float16)(b - (float)bh)});
-    }
-    uint4* dst = (uint4*)(T.k + tok * KROW + 32 * grp);
-    uint4* dlo = (uint4*)(T.klo + tok * KROW + 32 * grp);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      dst[q] = uint4{h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]};
-      dlo[q] = uint4{l[4 * q], l[4 * q + 1], l[4 * q + 2], l[4 * q + 3]};
+    if (4 * D % NT != 0 && c >= 4 * D) break;
+    const int k = c % D / NG, grp = c % NG;  // slots 0..15 of K, then of V
+    const int tok = 16 * (c / D) + (k & 15);
+    const uint32_t w = t0 + tok < total ? S.par[i] : 0u;
+    if (k < 16) {
+      Z.sk[grp * 64 + tok] = half_lo(w) * 16777216.0f;
+      const _Float16 z = __builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+      Z.z[tok * Int4Params<D>::ZROW + grp] = z;
+      Z.z[tok * Int4Params<D>::ZROW + NG + grp] = z;
+    } else {
+      Z.sv[grp * 64 + tok] = float2{half_lo(w) * kInt4VDown, half_hi(w) * kInt4VDown};
     }
   }
+}
+
+// Dim (within its chunk of 8) that element e of a staged K row holds: a
+// dword's nibbles leave as the pairs (0, 4), (1, 5), (2, 6), (3, 7).
+__device__ __forceinline__ constexpr int int4_dim(int e) { return (e >> 1) + 4 * (e & 1); }
+
+template <int D, int NT>
+__device__ __forceinline__ void stage_store4(const TileStage4<D, NT>& S, PrefillTile<D>& T,
+                                             const Int4Params<D>& Z, int tid) {
+  constexpr int KROW = PrefillTile<D>::KROW;
+  constexpr int VROW = PrefillTile<D>::VROW;
 #pragma unroll
-  for (int i = 0; i < TileStage4<D, NT>::VC; ++i) {
+  for (int i = 0; i < TileStage4<D, NT>::N; ++i) {
     const int c = tid + NT * i;
-    if (c >= TileStage4<D, NT>::VN) break;
+    if (4 * D % NT != 0 && c >= 4 * D) break;
     const int cb = c / D;
-    const int d = c % D;
-    const uint32_t w[2] = {S.vc[i].x, S.vc[i].y};
-    float val[16];
+    const int cc = c % D;
+    {
+      const int tok = 16 * cb + cc / (D / 16);
+      uint4* dst = (uint4*)(T.k + tok * KROW + 16 * (cc % (D / 16)));
+      const uint32_t ws[2] = {S.kc[i].x, S.kc[i].y};
 #pragma unroll
-    for (int sl = 0; sl < 16; ++sl) {
-      const uint32_t nib = (w[sl >> 3] >> (4 * (sl & 7))) & 0xF;
-      const bool valid = t0 + 16 * cb + sl < total;
-      // exact power-of-two scaling after the f32 dequantisation
-      val[sl] = valid ? ((float)nib * half_lo(S.vp[i][sl]) + half_hi(S.vp[i][sl])) * kInt4VDown
-                      : 0.0f;
+      for (int q = 0; q < 2; ++q)
+        dst[q] = uint4{ws[q] & 0x000F000Fu, (ws[q] >> 4) & 0x000F000Fu,
+                       (ws[q] >> 8) & 0x000F000Fu, (ws[q] >> 12) & 0x000F000Fu};
     }
+    const int d = cc;
     // slot s of page cb: k step cb>>1, group s>>2, element (cb&1)*4 + (s&3)
     _Float16* row = T.v + ((size_t)(cb >> 1) * D + d) * VROW;
     const int half = (cb & 1) * 4;
+    const float2* par = Z.sv + (d / 32) * 64 + 16 * cb;
+    const uint32_t ws[2] = {S.vc[i].x, S.vc[i].y};
 #pragma unroll
     for (int gg = 0; gg < 4; ++gg) {
-      const uint32_t h01 = __builtin_bit_cast(
-          uint32_t, v2h{(_Float16)val[4 * gg], (_Float16)val[4 * gg + 1]});
-      const uint32_t h23 = __builtin_bit_cast(
-          uint32_t, v2h{(_Float16)val[4 * gg + 2], (_Float16)val[4 * gg + 3]});
-      *(uint2*)(row + gg * 8 + half) = uint2{h01, h23};
+      const uint32_t w = ws[gg >> 1] >> (16 * (gg & 1));
+      const float4 p01 = *(const float4*)(par + 4 * gg);
+      const float4 p23 = *(const float4*)(par + 4 * gg + 2);
+      const v2h h01 = {(_Float16)__builtin_fmaf((float)(w & 0xF), p01.x, p01.y),
+                       (_Float16)__builtin_fmaf((float)((w >> 4) & 0xF), p01.z, p01.w)};
+      const v2h h23 = {(_Float16)__builtin_fmaf((float)((w >> 8) & 0xF), p23.x, p23.y),
+                       (_Float16)__builtin_fmaf((float)((w >> 12) & 0xF), p23.z, p23.w)};
+      *(uint2*)(row + gg * 8 + half) =
+          uint2{__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23)};
     }
   }
+}
+
+// ---- the query rows of a wave ----------------------------------------------
+// Lane (r, g) holds dims 32ks + 8g .. +7 of row r of each block, k steps ks.
+// The rows and their RoPE table entries come in 16-byte pieces (8-byte ones
+// where a 168-wide bf16 row is only that aligned); inputs that are not 16-byte
+// aligned (q_vec = 0) take one dword per element. Element by element, this
+// prologue took 19 us of every workgroup at head_dim 128 (2 x 32 query and
+// 128 table loads per lane); in pieces 3.2.
+template <int D, int RB>
+__device__ __forceinline__ void load_q_rows(const PrefillParams& p, const size_t (&row)[RB], int g,
+                                            float (&x)[RB][D / 32][8]) {
+  constexpr int KS = D / 32;
+  const bool bf16 = p.q_dtype == kDtypeBf16;
+  if (!p.q_vec) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int dl = logical_dim<D>(32 * ks + 8 * g + e);
+          x[rb][ks][e] = load_elem(p.q, row[rb] + (dl < 0 ? 0 : dl), p.q_dtype);
+          if (dl < 0) x[rb][ks][e] = 0.0f;
+        }
+    return;
+  }
+  // 4 dims from c0 on are all real or all padding (of the stored width 192)
+  auto four = [&](int rb, int c0) { return row[rb] + max(logical_dim<D>(c0), 0); };
+  if (bf16) {
+    uint2 w[RB][KS][2];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int c0 = 32 * ks + 8 * g;
+        if constexpr (kLogicalDim<D> == D) {
+          const uint4 v = *(const uint4*)((const uint16_t*)p.q + row[rb] + c0);
+          w[rb][ks][0] = uint2{v.x, v.y}, w[rb][ks][1] = uint2{v.z, v.w};
+        } else {
+          w[rb][ks][0] = *(const uint2*)((const uint16_t*)p.q + four(rb, c0));
+          w[rb][ks][1] = *(const uint2*)((const uint16_t*)p.q + four(rb, c0 + 4));
+        }
+      }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint2 v = w[rb][ks][e >> 2];
+          const uint32_t u = (e & 2) ? v.y : v.x;
+          x[rb][ks][e] = __uint_as_float((e & 1) ? u & 0xFFFF0000u : u << 16);
+        }
+  } else {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float4 v = *(const float4*)((const float*)p.q + four(rb, 32 * ks + 8 * g + 4 * h));
+          x[rb][ks][4 * h] = v.x, x[rb][ks][4 * h + 1] = v.y;
+          x[rb][ks][4 * h + 2] = v.z, x[rb][ks][4 * h + 3] = v.w;
+        }
+  }
+  if constexpr (kLogicalDim<D> != D) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (logical_dim<D>(32 * ks + 8 * g + e) < 0)
+#pragma unroll
+          for (int rb = 0; rb < RB; ++rb) x[rb][ks][e] = 0.0f;
+  }
+}
+
+// RoPE of those rows at positions pos. Split-half partners (d +- D/2) are the
+// same lane's chunk ks +- KS/2, interleaved ones (d ^ 1) its neighbours.
+template <int D, int RB>
+__device__ __forceinline__ void rope_q_rows(const PrefillParams& p, const int (&pos)[RB], int g,
+                                            float (&x)[RB][D / 32][8]) {
+  constexpr int KS = D / 32, KH = KS / 2;
+  constexpr int HL = kLogicalDim<D> / 2;  // table entries per position
+  if (!p.interleaved) {
+    float4 c[RB][KH][2], s[RB][KH][2];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ks = 0; ks < KH; ++ks)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int e0 = 32 * ks + 8 * g + 4 * h;
+          const size_t at = (size_t)pos[rb] * HL + (e0 < HL ? e0 : 0);
+          c[rb][ks][h] = *(const float4*)(p.cos_cache + at);
+          s[rb][ks][h] = *(const float4*)(p.sin_cache + at);
+        }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int ks = 0; ks < KH; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float4 cv = c[rb][ks][e >> 2], sv = s[rb][ks][e >> 2];
+          const float ce = (e & 2) ? ((e & 1) ? cv.w : cv.z) : ((e & 1) ? cv.y : cv.x);
+          const float se = (e & 2) ? ((e & 1) ? sv.w : sv.z) : ((e & 1) ? sv.y : sv.x);
+          const float x0 = x[rb][ks][e], x1 = x[rb][ks + KH][e];
+          // padding dims stay 0 whatever the table holds
+          const bool real = 32 * ks + 8 * g + e < HL;
+          x[rb][ks][e] = real ? rope_elem(ce, se, x0, x1, true) : 0.0f;
+          x[rb][ks + KH][e] = real ? rope_elem(ce, se, x1, x0, false) : 0.0f;
+        }
+    return;
+  }
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int dl = logical_dim<D>(32 * ks + 8 * g + 4 * h);  // 4 dims, 2 entries
+        const size_t at = (size_t)pos[rb] * HL + (dl < 0 ? 0 : dl >> 1);
+        const float2 c = *(const float2*)(p.cos_cache + at);
+        const float2 s = *(const float2*)(p.sin_cache + at);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const float ce = i ? c.y : c.x, se = i ? s.y : s.x;
+          const float x0 = x[rb][ks][4 * h + 2 * i], x1 = x[rb][ks][4 * h + 2 * i + 1];
+          x[rb][ks][4 * h + 2 * i] = dl < 0 ? 0.0f : rope_elem(ce, se, x0, x1, true);
+          x[rb][ks][4 * h + 2 * i + 1] = dl < 0 ? 0.0f : rope_elem(ce, se, x1, x0, false);
+        }
+      }
 }
 
 // RB row blocks of 16 attention rows per wave: 2 up to head_dim 128, 1 at
@@ -415,20 +551,22 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   constexpr int RB = D > 128 ? 1 : 2;
   constexpr int QT = 16 * RB * NW / G;  // query positions per workgroup
   constexpr bool INT4 = Q == kQuantInt4;
-  typedef PrefillTile<D, INT4> Tile;
+  typedef PrefillTile<D> Tile;
   constexpr int KROW = Tile::KROW;
   constexpr int VROW = Tile::VROW;
-  constexpr int HALF = D / 2;
   constexpr int DL = kLogicalDim<D>;  // the caller's rows (q, out)
-  constexpr int HL = DL / 2;          // table entries per position
 
   // int8 at head_dim <= 128 keeps four tiles in LDS and computes two per
   // barrier (4 x 38.4 KB at 128); int4 up to 128 and int8 at 256 keep two;
-  // int4 at 256 (an f16 hi + lo K tile and the V tile, 109 KB) keeps one and
-  // stages behind a second barrier
+  // int4 at 256 (75 KB a tile, and the parameters) keeps one and stages behind
+  // a second barrier
   constexpr int NSLOT = (!INT4 && D <= 128) ? 4 : ((INT4 && D > 128) ? 1 : 2);
   constexpr int PER_BARRIER = NSLOT == 4 ? 2 : 1;
   __shared__ Tile sT[NSLOT];
+  __shared__ Int4Params<INT4 ? D : 32> sZ[INT4 ? 3 : 1];
+  // int4: each lane's query operand of the zero points' k step (registers are
+  // what this kernel is short of; a lane reads back its own)
+  __shared__ v8h sQZ[INT4 ? NW * RB : 1][64];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -494,91 +632,140 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   typedef typename std::conditional<INT4, TileStage4<D, NT>, TileStage<D, NT>>::type Stage;
   Stage S;
   StagePages<D, NT, INT4> pages;  // page ids of the next tile to load
-  auto load_stage = [&](int t0) {
-    if constexpr (INT4)
-      stage_load4<D, NT>(S, p, pages, kvh, t0, tid);
-    else
-      stage_load<D, NT>(S, p, pages, kvh, t0, tid);
-  };
-  auto store_stage = [&](Tile& T, int t0) {
-    if constexpr (INT4)
-      stage_store4<D, NT>(S, T, t0, total, tid);
-    else
-      stage_store<D, NT>(S, T, t0, total, tid);
+  StagePages<D, NT, INT4> pages2;  // int4: of the tile after it, whose parameters load with it
+  auto zslot = [&](int tile) -> auto& { return sZ[INT4 ? (uint32_t)(tile - t_first) % 3u : 0]; };
+  // loads tile `tile` (and the parameters of the next one), then the page ids
+  // of the tiles after
+  auto load_stage = [&](int tile) {
+    if constexpr (INT4) {
+      stage_load4<D, NT>(S, p, pages, kvh, tid);
+      params_load4<D, NT>(S, p, pages2, kvh, tid);
+      pages = pages2;
+      pages2.load(pt, tile + 2, last_page, tid);
+    } else {
+      stage_load<D, NT>(S, p, pages, kvh, tile * 64, tid);
+      pages.load(pt, tile + 1, last_page, tid);
+    }
   };
   auto slot = [&](int tile) -> Tile& { return sT[(tile - t_first) & (NSLOT - 1)]; };
+  auto store_stage = [&](int tile) {
+    if constexpr (INT4) {
+      params_store4<D, NT>(S, zslot(tile + 1), (tile + 1) * 64, total, tid);
+      stage_store4<D, NT>(S, slot(tile), zslot(tile), tid);
+    } else {
+      stage_store<D, NT>(S, slot(tile), tile * 64, total, tid);
+    }
+  };
   pages.load(pt, t_first, last_page, tid);
-  load_stage(t_first * 64);
-  pages.load(pt, t_first + 1, last_page, tid);
+  if constexpr (INT4) {
+    // the first tile's parameters, and the zeros of the z rows
+    pages2.load(pt, t_first + 1, last_page, tid);
+    params_load4<D, NT>(S, p, pages, kvh, tid);
+    constexpr int ZR = Int4Params<D>::ZROW, NZ = 2 * (D / 32);
+    for (int e = tid; e < 3 * 64 * (32 - NZ); e += NT)
+      sZ[e / (64 * (32 - NZ))].z[e / (32 - NZ) % 64 * ZR + NZ + e % (32 - NZ)] = (_Float16)0.0f;
+    params_store4<D, NT>(S, zslot(t_first), t_first * 64, total, tid);
+  }
+  load_stage(t_first);
 
   // ---- Q^T operand: rows R = wave*32 + rb*16 + r -> (position, head) -------
   // RoPE(q) * scale * log2(e) as an f16 pair hi + lo (~22 bits: a score's
   // rounding error stays ~2^-20 of its largest term, outlier channels
   // included); lane (r, g) holds dims 32ks + 8g .. +7
   v8h qB[RB][KS], qL[RB][KS];
-  int qpos[RB];  // absolute position of the row (clamped for dead rows)
+  int qpos[RB];  // absolute position of the row (-1 for dead rows)
+  float qz_up[RB];  // int4: factor of the zero points' product (uniform)
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int R = wave * (16 * RB) + rb * 16 + r;
-    const int il = q0 + R / G;
-    const int hq = kvh * G + R % G;
-    const int i = il < p.sq ? il : p.sq - 1;
-    const int pos = past + i;
-    qpos[rb] = il < p.sq ? pos : -1;
-    const size_t qbase = (((size_t)b * p.sq + i) * Hq + hq) * DL;
-    float x[KS][8];
+  for (int rb = 0; rb < RB; ++rb) qz_up[rb] = 1.0f;
+  {
+    int pos[RB];
+    size_t qrow[RB];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int rb = 0; rb < RB; ++rb) {
+      const int R = wave * (16 * RB) + rb * 16 + r;
+      const int il = q0 + R / G;
+      const int i = il < p.sq ? il : p.sq - 1;
+      pos[rb] = past + i;
+      qpos[rb] = il < p.sq ? pos[rb] : -1;
+      qrow[rb] = (((size_t)b * p.sq + i) * Hq + kvh * G + R % G) * DL;
+    }
+    float x[RB][KS][8];
+    load_q_rows<D, RB>(p, qrow, g, x);
+    if (p.do_rotary) rope_q_rows<D, RB>(p, pos, g, x);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        // stored dim -> the caller's dim (padding dims of the stored width
-        // 192 are 0)
-        const int dl = logical_dim<D>(32 * ks + 8 * g + e);
-        x[ks][e] = load_elem(p.q, qbase + (dl < 0 ? 0 : dl), p.q_dtype);
-        if (dl < 0) x[ks][e] = 0.0f;
-      }
-    if (p.do_rotary) {
-      // partners: interleaved d ^ 1 (same chunk); split-half d +- D/2 (chunk
-      // ks +- KS/2, the same lane)
-      float y[KS][8];
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int d = 32 * ks + 8 * g + e;
-          const int dl = logical_dim<D>(d);
-          const bool first = p.interleaved ? (e & 1) == 0 : d < HALF;
-          const int pi = dl < 0 ? 0 : (p.interleaved ? (dl >> 1) : (first ? d : d - HALF));
-          const float partner = p.interleaved ? x[ks][e ^ 1] : x[(ks + KS / 2) % KS][e];
-          y[ks][e] = rope_elem(p.cos_cache[(size_t)pos * HL + pi],
-                               p.sin_cache[(size_t)pos * HL + pi], x[ks][e], partner, first);
-          if (dl < 0) y[ks][e] = 0.0f;
+          float xs = x[rb][ks][e] * p.scale_log2;
+          // one rounded product feeds both halves of the split
+          __asm__("" : "+v"(xs));
+          const _Float16 hi = (_Float16)xs;
+          qB[rb][ks][e] = hi;
+          qL[rb][ks][e] = (_Float16)(xs - (float)hi);
         }
+    if constexpr (INT4) {
+      // the sums of a group's query elements (as they enter the product), for
+      // the zero points: k elements [0, NG) their binary16 hi, [NG, 2 NG) lo
+      constexpr int NG = KS;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
+      for (int rb = 0; rb < RB; ++rb) {
+        float sum[NG];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[ks][e] = y[ks][e];
-    }
+        for (int ks = 0; ks < KS; ++ks) {
+          sum[ks] = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+          for (int e = 0; e < 8; ++e) sum[ks] += (float)qB[rb][ks][e] + (float)qL[rb][ks][e];
+          sum[ks] = xgroup_sum(sum[ks]);
+        }
+        // a sum of 32 binary16 values may pass the type's range: the sums then
+        // go in 2^-5 smaller
+        float most = 0.0f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float xs = x[ks][e] * p.scale_log2;
-        // one rounded product feeds both halves of the split
-        __asm__("" : "+v"(xs));
-        const _Float16 hi = (_Float16)xs;
-        qB[rb][ks][e] = hi;
-        qL[rb][ks][e] = (_Float16)(xs - (float)hi);
+        for (int ks = 0; ks < NG; ++ks) most = fmaxf(most, fabsf(sum[ks]));
+        const bool shrink = __builtin_amdgcn_ballot_w64(most > 32768.0f) != 0;
+        if (shrink) qz_up[rb] = 32.0f;
+        const float down = shrink ? 0.03125f : 1.0f;
+        v8h qz;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          // element 8g + e of the k step
+          float v = 0.0f;
+#pragma unroll
+          for (int k = 0; k < 2 * NG; ++k) {
+            if (k % 8 != e) continue;
+            float t = sum[k % NG] * down;
+            __asm__("" : "+v"(t));
+            const float hi = (float)(_Float16)t;
+            v = g == k / 8 ? (k < NG ? hi : t - hi) : v;
+          }
+          qz[e] = (_Float16)v;
+        }
+        sQZ[wave * RB + rb][lane] = qz;
+        // the staged K rows' order within a chunk of 8 dims
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          v8h hi, lo;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) hi[e] = qB[rb][ks][int4_dim(e)], lo[e] = qL[rb][ks][int4_dim(e)];
+          qB[rb][ks] = hi, qL[rb][ks] = lo;
+        }
       }
+    }
   }
 
-  store_stage(slot(t_first), t_first * 64);
+  if constexpr (INT4) __syncthreads();  // the first tile's parameters
+  store_stage(t_first);
   if (PER_BARRIER == 2 && t_first + 1 < t_last) {
-    load_stage((t_first + 1) * 64);
-    pages.load(pt, t_first + 2, last_page, tid);
-    store_stage(slot(t_first + 1), (t_first + 1) * 64);
+    load_stage(t_first + 1);
+    store_stage(t_first + 1);
   }
   __syncthreads();
+
+  // a wave whose rows all lie past the chunk only helps to stage the tiles
+  const bool wave_live =
+      __builtin_amdgcn_readfirstlane(q0 + wave * (16 * RB) / G < p.sq ? 1 : 0) != 0;
 
   // ---- online softmax state ----------------------------------------------------
   // m_run: the row's reference point (set from its first visible keys; 0 only
@@ -623,11 +810,92 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
     }
     const float lc = (float)dexp;
 
+    // keys past a row's position or before its window: -inf
+    auto mask = [&](float (&s)[RB][4][4]) __attribute__((always_inline)) {
+      if (tile >= full_tiles || tile < lo_full) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+          for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int t = t0 + 16 * cb + 4 * g + e;
+              const bool vis = t <= qpos[rb] && (W <= 0 || t > qpos[rb] - W);
+              s[rb][cb][e] = vis ? s[rb][cb][e] : -INFINITY;
+            }
+      }
+    };
     // S^T for both row blocks: 4 column blocks of 16 tokens; k steps outer so
     // that eight independent accumulation chains interleave on the MFMA pipe.
     // s holds each score relative to its row's reference point:
     // s = <q', k> * s_k - m_run + dexp (masked keys: -inf)
     auto scores = [&](float (&s)[RB][4][4]) __attribute__((always_inline)) {
+      if constexpr (INT4) {
+        // the zero points' k step on top of -m_run, then a group at a time
+        // (two of the four token blocks: their products, then, with the next
+        // pair's in flight, the scaled sums)
+        const auto& Z = zslot(tile);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          const v8h qz = sQZ[wave * RB + rb][lane];
+#pragma unroll
+          for (int cb = 0; cb < 4; ++cb) {
+            const v8h zf = *(const v8h*)(Z.z + (16 * cb + r) * Int4Params<D>::ZROW + 8 * g);
+            const float m = qz_up[rb] == 1.0f ? -m_run[rb] : 0.0f;
+            const v4f z = __builtin_amdgcn_mfma_f32_16x16x32_f16(zf, qz, v4f{m, m, m, m}, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[rb][cb][e] = z[e];
+          }
+          if (qz_up[rb] != 1.0f) {
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                s[rb][cb][e] = __builtin_fmaf(s[rb][cb][e], qz_up[rb], -m_run[rb]);
+          }
+        }
+        v4f c[2][RB];
+        auto products = [&](int i) {
+          const int ks = i >> 1, c0 = 2 * (i & 1);
+          v8h kf[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            kf[j] = *(const v8h*)(T.k + (16 * (c0 + j) + r) * KROW + 8 * g + 32 * ks);
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+              c[j][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  kf[j], qB[rb][ks], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+              c[j][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[j], qL[rb][ks],
+                                                                       c[j][rb], 0, 0, 0);
+        };
+        auto scaled = [&](int i) {
+          const int ks = i >> 1, c0 = 2 * (i & 1);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const float4 sv = *(const float4*)(Z.sk + 64 * ks + 16 * (c0 + j) + 4 * g);
+            const float sk[4] = {sv.x, sv.y, sv.z, sv.w};
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                s[rb][c0 + j][e] = __builtin_fmaf(c[j][rb][e], sk[e], s[rb][c0 + j][e]);
+          }
+        };
+#pragma unroll
+        for (int i = 0; i < 2 * KS; ++i) {
+          products(i);
+          scaled(i);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        mask(s);
+        return;
+      }
       v4f c[4][RB];
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb)
@@ -660,45 +928,21 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
 #pragma unroll
           for (int rb = 0; rb < RB; ++rb)
             c[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[ks & 1][cb], qL[rb][ks], c[cb][rb], 0, 0, 0);
-        if constexpr (INT4) {
-#pragma unroll
-          for (int cb = 0; cb < 4; ++cb) {
-            const v8h al = *(const v8h*)(T.klo + (16 * cb + r) * KROW + 8 * g + 32 * ks);
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-              c[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, qB[rb][ks], c[cb][rb], 0, 0, 0);
-          }
-        }
       }
       float mref[RB];
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) mref[rb] = INT4 ? m_run[rb] : m_run[rb] - lc;
+      for (int rb = 0; rb < RB; ++rb) mref[rb] = m_run[rb] - lc;
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) {
-        float skx[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-        if constexpr (!INT4) {
-          const float4 skv = *(const float4*)(T.sk + 16 * cb + 4 * g);
-          skx[0] = skv.x, skx[1] = skv.y, skx[2] = skv.z, skx[3] = skv.w;
-        }
+        const float4 skv = *(const float4*)(T.sk + 16 * cb + 4 * g);
+        const float skx[4] = {skv.x, skv.y, skv.z, skv.w};
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            s[rb][cb][e] = INT4 ? c[cb][rb][e] - mref[rb]
-                                : __builtin_fmaf(c[cb][rb][e], skx[e], -mref[rb]);
+            s[rb][cb][e] = __builtin_fmaf(c[cb][rb][e], skx[e], -mref[rb]);
       }
-      if (tile >= full_tiles || tile < lo_full) {
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-          for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int t = t0 + 16 * cb + 4 * g + e;
-              const bool vis = t <= qpos[rb] && (W <= 0 || t > qpos[rb] - W);
-              s[rb][cb][e] = vis ? s[rb][cb][e] : -INFINITY;
-            }
-      }
+      mask(s);
     };
     // s -> p = exp2(s) in place; rsum = the row's sum over the tile
     auto weights = [&](float (&s)[RB][4][4], float (&rsum)[RB]) __attribute__((always_inline)) {
@@ -819,7 +1063,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
       // the MFMAs that consume them (the scheduler fence keeps each read ahead
       // of its consumer by that many MFMA pairs, so the LDS latency is covered)
       constexpr int NV = 2 * JB;
-      constexpr int PF = INT4 ? kVPrefetchInt4 : kVPrefetch;
+      constexpr int PF = kVPrefetch;
       v8h vf[NV];
 #pragma unroll
       for (int i = 0; i < PF && i < NV; ++i) vf[i] = vfrag(i);
@@ -893,14 +1137,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
         break;
       }
       const bool more = tile + 1 < t_last;
-      if (more) {
-        load_stage((tile + 1) * 64);
-        pages.load(pt, tile + 2, last_page, tid);
-      }
-      process(sT[0], tile);
+      if (more) load_stage(tile + 1);
+      if (wave_live) process(sT[0], tile);
       __syncthreads();
       if (more) {
-        store_stage(sT[0], (tile + 1) * 64);
+        store_stage(tile + 1);
         __syncthreads();
       }
     }
@@ -920,12 +1161,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
         if (tt < t_last) {
           const int nxt = tt + PER_BARRIER;
           const bool more = nxt < t_last;
-          if (more) {
-            load_stage(nxt * 64);
-            pages.load(pt, nxt + 1, last_page, tid);  // consumed by the next stage
-          }
-          process(slot(tt), tt);
-          if (more) store_stage(slot(nxt), nxt * 64);
+          if (more) load_stage(nxt);
+          if (wave_live) process(slot(tt), tt);
+          if (more) store_stage(nxt);
         }
       }
       __syncthreads();
@@ -1003,9 +1241,11 @@ hipError_t launch_pass(const PrefillParams& p, int group, hipStream_t st) {
 // The fast pass, then (int8) the precise pass over the workgroups it flagged.
 template <int D, int NW, int Q>
 hipError_t launch_dn(const PrefillParams& p, int group, hipStream_t st) {
-  hipError_t e = launch_pass<D, NW, Q, false>(p, group, st);
-  if (e != hipSuccess || Q != kQuantInt8) return e;
-  return launch_pass<D, NW, Q, true>(p, group, st);
+  const hipError_t e = launch_pass<D, NW, Q, false>(p, group, st);
+  if constexpr (Q == kQuantInt8)
+    return e != hipSuccess ? e : launch_pass<D, NW, Q, true>(p, group, st);
+  else
+    return e;
 }
 
 // 8 waves (256 rows) per workgroup: the staged K/V tile serves twice the rows

@@ -1101,6 +1101,7 @@ SAI_API sai_status sai_gqa_prefill(sai_ctx* ctx, sai_kvcache* c, int32_t layer, 
   sai::PrefillParams p{};
   p.q = q;
   p.q_dtype = dtype;
+  p.q_vec = ((uintptr_t)q & 15u) == 0;
   p.out = out;
   p.out_bf16 = out_dtype == SAI_DTYPE_BF16 ? 1 : 0;
   p.pool = c->pools[layer];

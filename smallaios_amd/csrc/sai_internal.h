@@ -237,6 +237,7 @@ struct DecodeParams {
 struct PrefillParams {
   const void* q;  // [batch, sq, Hq*D]
   int q_dtype;
+  int q_vec;  // q is 16-byte aligned
   void* out;     // [batch, sq, Hq*D], f32 or (out_bf16) bf16
   int out_bf16;
   const uint8_t* pool;
