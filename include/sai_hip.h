@@ -459,9 +459,9 @@ int32_t sai_set_decode_waves(sai_ctx* ctx, int32_t waves);
  * combine kernel, 1 = the last workgroup of a (sequence, kv head) merges
  * in-kernel (the partials are handed over with agent-scope stores and loads,
  * one ticket counter per (sequence, kv head)), 2 = automatic (the default:
- * in-kernel when every sequence of the launch has the same split count, else
- * the combine kernel). Returns the previous value; other values are
- * ignored. */
+ * in-kernel up to 16 splits per sequence, when every sequence has the same
+ * split count or the launch is at most two workgroups per CU, else the
+ * combine kernel). Returns the previous value; other values are ignored. */
 int32_t sai_set_decode_merge(sai_ctx* ctx, int32_t in_kernel);
 /* Tile order of the int8 decode kernel and the TurboQuant attention. Fixed:
  * each wave of a workgroup takes tiles w, w + waves, ..., so repeated calls on

@@ -116,6 +116,19 @@ __device__ __forceinline__ void store_partial(float* a, float v) {
 __device__ __forceinline__ float load_partial(const float* a) {
   return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Two neighbouring floats at once (8-byte aligned: a partial's rows hold an
+// even number of floats).
+__device__ __forceinline__ void store_partial2(float* a, float v0, float v1) {
+  __hip_atomic_store((unsigned long long*)a,
+                     (unsigned long long)__float_as_uint(v0) |
+                         ((unsigned long long)__float_as_uint(v1) << 32),
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_partial2(const float* a) {
+  const unsigned long long w = __hip_atomic_load((const unsigned long long*)a, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+  return float2{__uint_as_float((uint32_t)w), __uint_as_float((uint32_t)(w >> 32))};
+}
 // Every vector memory access of this wave issued so far has completed (on
 // gfx9 vmcnt counts stores until they are acknowledged); also a compiler
 // barrier, so no store is moved past it.
@@ -164,21 +177,112 @@ __device__ __forceinline__ void merge_partials(const float* ph, size_t stride, i
   }
 }
 
-// merge_partials with the batch width picked from the split count: all of a
-// (head, dim) entry's splits in one round trip up to 32 splits (each round
-// trip to partials written on other XCDs costs a full memory latency).
-__device__ __forceinline__ void merge_all_splits(const float* ph, size_t stride, int d,
-                                                 int nsplit, float& M, float& Ls, float& O) {
-  if (nsplit <= 2)
-    merge_partials<2>(ph, stride, d, nsplit, -1, M, Ls, O);
-  else if (nsplit <= 4)
-    merge_partials<4>(ph, stride, d, nsplit, -1, M, Ls, O);
+// The merge of a (sequence, kv head)'s nsplit partials by one workgroup of NT
+// threads: p0 points at split 0's block [G][m, l, o[D]], `stride` floats to
+// the next split's. A thread takes pairs of neighbouring dims; the loads of C
+// splits for all its pairs go out together with the (m, l) of those splits,
+// which reach the other threads through LDS (sm: C * G float2). Every load of
+// partials written on other XCDs is a full memory latency, so what counts is
+// the number of dependent rounds: one per C splits, whatever the entries per
+// thread. (One entry after the other, each loading its own m and l, took a
+// round per entry: 1 x 16384 in 32 splits, 8Q/1KV, D = 128, 30.1 us per step,
+// in one round per 16 splits 22.6; 1 x 8192 in 16, 32Q/8KV, 15.8 -> 13.9; the
+// Gemma 3 4B window layer in 5, 16.9 -> 16.0.) The result does not depend on
+// which workgroup merges.
+// store(head, dim, v0, v1) takes dims dim, dim + 1.
+template <int D, int G, int NT, int C, class F>
+__device__ __forceinline__ void merge_splits_by(const float* p0, size_t stride, int nsplit,
+                                                float2* sm, F&& store) {
+  constexpr int E = G * D / 2;  // pairs
+  constexpr int PER = (E + NT - 1) / NT;
+  const int tid = threadIdx.x;
+  float M[PER], L[PER], O0[PER], O1[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    M[k] = -INFINITY;
+    L[k] = O0[k] = O1[k] = 0.0f;
+  }
+  for (int s0 = 0; s0 < nsplit; s0 += C) {
+    const int n = min(C, nsplit - s0);
+    const float* ps = p0 + (size_t)s0 * stride;
+    float2 o[PER][C];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = min(tid + k * NT, E - 1), hd = e / (D / 2), d = 2 * (e % (D / 2));
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        o[k][i] = load_partial2(ps + (size_t)min(i, n - 1) * stride + hd * (D + 2) + 2 + d);
+    }
+    for (int t = tid; t < C * G; t += NT) {
+      const int i = t / G;
+      const float2 ml = load_partial2(ps + (size_t)min(i, n - 1) * stride + (t % G) * (D + 2));
+      sm[t] = i < n ? ml : float2{-INFINITY, 0.0f};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int hd = min(tid + k * NT, E - 1) / (D / 2);
+      float2 ml[C];  // read together: no branch between the LDS reads
+#pragma unroll
+      for (int i = 0; i < C; ++i) ml[i] = sm[i * G + hd];
+      float mb = M[k];
+#pragma unroll
+      for (int i = 0; i < C; ++i) mb = fmaxf(mb, ml[i].x);
+      // splits without a visible key (m = -inf, l = o = 0) weigh 2^-inf = 0
+      const float ref = mb == -INFINITY ? 0.0f : mb;
+      const float f0 = fast_exp2(M[k] - ref);
+      L[k] *= f0;
+      O0[k] *= f0;
+      O1[k] *= f0;
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const float f = fast_exp2(ml[i].x - ref);
+        L[k] += ml[i].y * f;
+        O0[k] += o[k][i].x * f;
+        O1[k] += o[k][i].y * f;
+      }
+      M[k] = mb;
+    }
+    if (s0 + C < nsplit) __syncthreads();  // sm is written again
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int e = tid + k * NT;
+    if (E % NT != 0 && e >= E) break;
+    store(e / (D / 2), 2 * (e % (D / 2)), L[k] > 0.0f ? O0[k] / L[k] : 0.0f,
+          L[k] > 0.0f ? O1[k] / L[k] : 0.0f);
+  }
+}
+
+// Rounds of 4, 8 or 16 splits by the split count (uniform).
+template <int D, int G, int NT, class F>
+__device__ __forceinline__ void merge_splits(const float* p0, size_t stride, int nsplit,
+                                             float2* sm, F&& store) {
+  if constexpr (G * D <= 64) {
+    // one wave holds every entry: a dim per lane, each reading its own (m, l),
+    // has no barrier in the way (int4, 1 x 4585, 8Q/8KV, D = 64, 9 splits:
+    // 11.96 against 12.60 us per step)
+    const int t = threadIdx.x;
+    if (t < G * D) {
+      float M = -INFINITY, L = 0.0f, O = 0.0f;
+      if (nsplit <= 4)
+        merge_partials<4>(p0, stride, t, nsplit, -1, M, L, O);
+      else if (nsplit <= 8)
+        merge_partials<8>(p0, stride, t, nsplit, -1, M, L, O);
+      else
+        merge_partials<16>(p0, stride, t, nsplit, -1, M, L, O);
+      const float v = L > 0.0f ? O / L : 0.0f;
+      const float next = __int_as_float(swap_pair(__float_as_int(v)));
+      if ((t & 1) == 0) store(0, t, v, next);
+    }
+    return;
+  }
+  if (nsplit <= 4)
+    merge_splits_by<D, G, NT, 4>(p0, stride, nsplit, sm, store);
   else if (nsplit <= 8)
-    merge_partials<8>(ph, stride, d, nsplit, -1, M, Ls, O);
-  else if (nsplit <= 16)
-    merge_partials<16>(ph, stride, d, nsplit, -1, M, Ls, O);
+    merge_splits_by<D, G, NT, 8>(p0, stride, nsplit, sm, store);
   else
-    merge_partials<32>(ph, stride, d, nsplit, -1, M, Ls, O);
+    merge_splits_by<D, G, NT, 16>(p0, stride, nsplit, sm, store);
 }
 
 // 16 consecutive elements (f32 or bf16) starting at element `off`; the
@@ -205,11 +309,14 @@ __device__ __forceinline__ void load16(const void* base, size_t off, int dtype, 
 
 // (sequence, split) of a decode workgroup and its split's length in 64-token
 // tiles. Uniform split count: direct mapping, splits of split_tokens.
-// Ragged: a prefix scan over the per-sequence split counts of seq_lens[b] +
-// pending tokens (in p.order when given), and a sequence's streamed tiles
-// dealt evenly to its splits (ceil(T / nsplit) each, the last split taking
-// the rest, never none), so no split is a short remainder. Returns b = -1
-// past the last work item.
+// Ragged: the host's table of work items (p.ordered), or for larger batches a
+// prefix scan over the per-sequence split counts of seq_lens[b] + pending
+// tokens; a sequence's streamed tiles are dealt evenly to its splits
+// (ceil(T / nsplit) each, the last split taking the rest, never none), so no
+// split is a short remainder. Returns b = -1 past the last work item.
+// (The scan waits for the lengths and then for six lane shuffles: 1.6 us of
+// every workgroup at 7 ragged sequences, whose step went from 18.8 to 16.7 us
+// with the table and the merge in the kernel.)
 __device__ __forceinline__ void decode_work_item(const DecodeParams& p, int work, int lane, int& b,
                                                  int& split, int& nsplit, int& split_base,
                                                  int& tps) {
@@ -223,10 +330,29 @@ __device__ __forceinline__ void decode_work_item(const DecodeParams& p, int work
     split_base = b * nsplit;
     return;
   }
+  if (p.ordered) {
+    // the host's table: no lengths, no scan, one round trip
+    for (int c0 = 0; c0 < p.batch; c0 += 64) {
+      const int i = min(c0 + lane, p.batch - 1);
+      const int end = p.item_end[i];
+      const int begin = i > 0 ? p.item_end[i - 1] : 0;
+      const int sb = p.order[i], tp = p.item_tps[i];
+      const unsigned long long m = __ballot(end > work);
+      if (m == 0) continue;
+      const int first = __ffsll((long long)m) - 1;
+      b = __builtin_amdgcn_readlane(sb, first);
+      split_base = __builtin_amdgcn_readlane(begin, first);
+      nsplit = __builtin_amdgcn_readlane(end, first) - split_base;
+      tps = __builtin_amdgcn_readlane(tp, first);
+      split = work - split_base;
+      return;
+    }
+    return;
+  }
   int base = 0;
   for (int c0 = 0; c0 < p.batch; c0 += 64) {
     const int bi = c0 + lane;
-    const int sb = bi < p.batch ? (p.ordered ? (int)p.order[bi] : bi) : 0;
+    const int sb = bi < p.batch ? bi : 0;
     const int Lb = bi < p.batch ? p.seq_lens[sb] + p.pending : 0;
     const int span = Lb - window_origin(Lb, p.window);
     const int n = (span + p.split_tokens - 1) / p.split_tokens;

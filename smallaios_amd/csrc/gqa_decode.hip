@@ -442,14 +442,23 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
   // waiting for it never waits for them
   int gq = 0;
   if (have_first) gq = grab_issue();
-  // The first tile's loads and the touch below are issued by every wave (a
-  // wave without a tile re-reads tile 0 of its split, which always exists):
-  // behind a branch, the compiler's wait counts for the query's loads would
-  // have to assume the branch was not taken and wait for these loads too.
+  WaveState<D, G> st;
+#pragma unroll
+  for (int ps = 0; ps < NP; ++ps) {
+    st.m_run[ps] = -INFINITY;
+    st.l_run[ps] = 0.0f;
+#pragma unroll
+    for (int jb = 0; jb < JB; ++jb) st.acc[ps][jb] = 0.0f;
+  }
+  __shared__ float sm_sc[NW][128];
+  // A wave without a tile goes straight to the merge (short sequences: it
+  // would only take issue slots from the waves that have one). Everything from
+  // the first tile's loads on is inside, so that no join lies between them and
+  // their uses (at a join the compiler waits for all loads of either path).
+  if (have_first) {
   TileRegs<D> TA;
-  const int first_ld = have_first ? first : 0;
   if constexpr (!BIG)
-    load_tile<D>(TA, p.pool, sm_pg, first_ld, p.num_pages, kvh, r, g, n_pages_split);
+    load_tile<D>(TA, p.pool, sm_pg, first, p.num_pages, kvh, r, g, n_pages_split);
   // Tile first + slots (the one this wave most likely takes next, never the
   // appender's; else the first tile again) is touched (one dword per 128-byte
   // line) so that it streams into L2 while the query is prepared, instead of
@@ -462,7 +471,7 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
 #pragma unroll
   for (int j = 0; j < kTouch; ++j) touch[j] = 0;
   if constexpr (!BIG) {
-    const int t1 = have_first && first + slots < pool_end ? first + slots : first_ld;
+    const int t1 = first + slots < pool_end ? first + slots : first;
 #pragma unroll
     for (int j = 0; j < kTouch; ++j) {
       const int line = min(lane + 64 * j, 4 * kLines - 1);
@@ -566,18 +575,8 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
     const float w0 = s0 * p.scale_log2;
     qw[ps] = tq == 0 ? w0 : (tq == 1 ? w0 * (1.0f / 254.0f) : (tq == 2 ? w0 * (1.0f / 64516.0f) : 0.0f));
   }
-  __shared__ float sm_sc[NW][128];
 
   // ---- stream the split's tiles, double-buffered --------------------------------
-  WaveState<D, G> st;
-#pragma unroll
-  for (int ps = 0; ps < NP; ++ps) {
-    st.m_run[ps] = -INFINITY;
-    st.l_run[ps] = 0.0f;
-#pragma unroll
-    for (int jb = 0; jb < JB; ++jb) st.acc[ps][jb] = 0.0f;
-  }
-
   // Ping-pong between two tile buffers: the next tile is taken and its load
   // issued before the current one is computed, so one tile is always in
   // flight; the loads inside the loop are unconditional once a tile is taken.
@@ -593,7 +592,7 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
   // (the index for the tile after next is asked for before the next tile's
   // loads are issued, for the same reason as above)
   if constexpr (D <= 128) {
-    if (have_first) {
+    {
       int cur = first;
       for (;;) {
         const int n1 = grab_value(gq);
@@ -620,7 +619,7 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
     // phase: the next tile's K (and scales) load as soon as this tile's QK is
     // issued, its V as soon as this tile's PV is (the last tile reloads
     // itself, so the code stays straight-line)
-    if (have_first) {
+    {
       int cur = first;
       ld(TA, cur);
       for (;;) {
@@ -640,10 +639,12 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
     }
   }
 
+  }  // have_first
+
   // ---- merge the NW waves of the workgroup --------------------------------------
   __shared__ float sm_m[NW][G];
   __shared__ float sm_l[NW][G];
-  __shared__ float sm_o[NW][G][D];
+  alignas(16) __shared__ float sm_o[NW][G][D];
 #pragma unroll
   for (int ps = 0; ps < NP; ++ps) {
     const int h = 4 * ps + (r >> 2);
@@ -659,41 +660,44 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
   __syncthreads();
 
   float* part = p.partials + ((size_t)(split_base + split) * p.kv_heads + kvh) * (G * (D + 2));
-  // (m, l, o) of this split for the (head, dim) entries t = threadIdx.x + k*64*NW
-  constexpr int PER = (G * D + 64 * NW - 1) / (64 * NW);
+  // (m, l, o) of this split for pairs of neighbouring dims, pair t =
+  // threadIdx.x + k*64*NW
+  constexpr int E = G * D / 2;
+  constexpr int PER = (E + 64 * NW - 1) / (64 * NW);
+  auto store_pair = [&](int hd, int d, float v0, float v1) {
+    const int dl = logical_dim<D>(d);  // -1: padding dims, not written
+    if (dl < 0) return;
+    const size_t at = ((size_t)b * Hq + kvh * G + hd) * DL + dl;
+    store_out(p.out, at, v0, p.out_bf16);
+    store_out(p.out, at + 1, v1, p.out_bf16);
+  };
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const int t = threadIdx.x + k * 64 * NW;
-    if (G * D % (64 * NW) != 0 && t >= G * D) break;
-    const int hd = t / D, d = t % D;
+    if (E % (64 * NW) != 0 && t >= E) break;
+    const int hd = t / (D / 2), d = 2 * (t % (D / 2));
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_m[w][hd]);
-    float Ls = 0.0f, O = 0.0f;
+    float Ls = 0.0f, O0 = 0.0f, O1 = 0.0f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       if (sm_m[w][hd] == -INFINITY) continue;
       const float f = fast_exp2(sm_m[w][hd] - M);
+      const float2 o = *(const float2*)&sm_o[w][hd][d];
       Ls += sm_l[w][hd] * f;
-      O += sm_o[w][hd][d] * f;
+      O0 += o.x * f;
+      O1 += o.y * f;
     }
-    const int dl = logical_dim<D>(d);  // -1: a padding dim, not written
+    float* row = part + hd * (D + 2);
     if (nsplit == 1) {
-      if (dl >= 0)
-        store_out(p.out, ((size_t)b * Hq + kvh * G + hd) * DL + dl, Ls > 0.0f ? O / Ls : 0.0f,
-                  p.out_bf16);
+      store_pair(hd, d, Ls > 0.0f ? O0 / Ls : 0.0f, Ls > 0.0f ? O1 / Ls : 0.0f);
     } else if (p.merge_in_kernel) {
-      store_partial(part + hd * (D + 2) + 2 + d, O);
-      if (d == 0) {
-        store_partial(part + hd * (D + 2), M);
-        store_partial(part + hd * (D + 2) + 1, Ls);
-      }
+      store_partial2(row + 2 + d, O0, O1);
+      if (d == 0) store_partial2(row, M, Ls);
     } else {
-      part[hd * (D + 2) + 2 + d] = O;
-      if (d == 0) {
-        part[hd * (D + 2)] = M;
-        part[hd * (D + 2) + 1] = Ls;
-      }
+      *(float2*)(row + 2 + d) = float2{O0, O1};
+      if (d == 0) *(float2*)row = float2{M, Ls};
     }
   }
   if (!p.merge_in_kernel) {
@@ -723,19 +727,7 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
   const float* p0 = p.partials + ((size_t)split_base * p.kv_heads + kvh) * (G * (D + 2));
   // every split's partial, this workgroup's own included, in split order: the
   // result does not depend on which workgroup finished last
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int t = threadIdx.x + k * 64 * NW;
-    if (G * D % (64 * NW) != 0 && t >= G * D) break;
-    const int hd = t / D, d = t % D;
-    float M = -INFINITY, Ls = 0.0f, O = 0.0f;
-    const float* ph = p0 + hd * (D + 2);
-    merge_all_splits(ph, stride, d, nsplit, M, Ls, O);
-    const int dl = logical_dim<D>(d);
-    if (dl >= 0)
-      store_out(p.out, ((size_t)b * Hq + kvh * G + hd) * DL + dl, Ls > 0.0f ? O / Ls : 0.0f,
-                p.out_bf16);
-  }
+  merge_splits<D, G, 64 * NW>(p0, stride, nsplit, (float2*)sm_o, store_pair);
   if (threadIdx.x == 0) reset_ticket(counter);
 }
 

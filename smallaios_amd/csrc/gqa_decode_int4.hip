@@ -575,7 +575,7 @@ __global__ __launch_bounds__(64 * NW, (kOneWavePerSimd<D, G>) ? 1 : 8 / NW) void
   __shared__ float sm_m[NW][G];
   __shared__ float sm_l[NW][G];
   __shared__ float sm_z[NW][G][NG];
-  __shared__ float sm_o[NW][G][D];
+  alignas(16) __shared__ float sm_o[NW][G][D];
 #pragma unroll
   for (int qd = 0; qd < HT; ++qd) {
     const int h = 4 * qd + hh;
@@ -597,33 +597,37 @@ __global__ __launch_bounds__(64 * NW, (kOneWavePerSimd<D, G>) ? 1 : 8 / NW) void
   __syncthreads();
 
   float* part = p.partials + ((size_t)(split_base + split) * p.kv_heads + kvh) * (G * (D + 2));
-  for (int t = threadIdx.x; t < G * D; t += 64 * NW) {
-    const int hd = t / D, d = t % D;
+  auto store_pair = [&](int hd, int d, float v0, float v1) {
+    const size_t at = ((size_t)b * Hq + kvh * G + hd) * D + d;
+    store_out(p.out, at, v0, p.out_bf16);
+    store_out(p.out, at + 1, v1, p.out_bf16);
+  };
+  // pairs of neighbouring dims
+  for (int t = threadIdx.x; t < G * D / 2; t += 64 * NW) {
+    const int hd = t / (D / 2), d = 2 * (t % (D / 2));
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_m[w][hd]);
-    float Ls = 0.0f, O = 0.0f;
+    float Ls = 0.0f, O0 = 0.0f, O1 = 0.0f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       if (sm_m[w][hd] == -INFINITY) continue;
       const float f = fast_exp2(sm_m[w][hd] - M);
+      const float2 o = *(const float2*)&sm_o[w][hd][d];
+      const float z = sm_z[w][hd][d >> 5];
       Ls += sm_l[w][hd] * f;
-      O += (sm_o[w][hd][d] + sm_z[w][hd][d >> 5]) * f;
+      O0 += (o.x + z) * f;
+      O1 += (o.y + z) * f;
     }
+    float* row = part + hd * (D + 2);
     if (nsplit == 1) {
-      store_out(p.out, ((size_t)b * Hq + kvh * G + hd) * D + d, Ls > 0.0f ? O / Ls : 0.0f, p.out_bf16);
+      store_pair(hd, d, Ls > 0.0f ? O0 / Ls : 0.0f, Ls > 0.0f ? O1 / Ls : 0.0f);
     } else if (p.merge_in_kernel) {
-      store_partial(part + hd * (D + 2) + 2 + d, O);
-      if (d == 0) {
-        store_partial(part + hd * (D + 2), M);
-        store_partial(part + hd * (D + 2) + 1, Ls);
-      }
+      store_partial2(row + 2 + d, O0, O1);
+      if (d == 0) store_partial2(row, M, Ls);
     } else {
-      part[hd * (D + 2) + 2 + d] = O;
-      if (d == 0) {
-        part[hd * (D + 2)] = M;
-        part[hd * (D + 2) + 1] = Ls;
-      }
+      *(float2*)(row + 2 + d) = float2{O0, O1};
+      if (d == 0) *(float2*)row = float2{M, Ls};
     }
   }
   if (!p.merge_in_kernel) {
@@ -650,13 +654,7 @@ __global__ __launch_bounds__(64 * NW, (kOneWavePerSimd<D, G>) ? 1 : 8 / NW) void
   if (!sm_last) return;
   const size_t stride = (size_t)p.kv_heads * (G * (D + 2));
   const float* p0 = p.partials + ((size_t)split_base * p.kv_heads + kvh) * (G * (D + 2));
-  for (int t = threadIdx.x; t < G * D; t += 64 * NW) {
-    const int hd = t / D, d = t % D;
-    float M = -INFINITY, Ls = 0.0f, O = 0.0f;
-    const float* ph = p0 + hd * (D + 2);
-    merge_all_splits(ph, stride, d, nsplit, M, Ls, O);
-    store_out(p.out, ((size_t)b * Hq + kvh * G + hd) * D + d, Ls > 0.0f ? O / Ls : 0.0f, p.out_bf16);
-  }
+  merge_splits<D, G, 64 * NW>(p0, stride, nsplit, (float2*)sm_o, store_pair);
   if (threadIdx.x == 0) reset_ticket(counter);
 }
 

@@ -861,6 +861,23 @@ sai_status launch_decode(sai_ctx* ctx, sai_kvcache* c, int32_t layer, const void
     if (split < 512 && (c->desc.quant == SAI_KV_INT8 ? (max_len <= 512 || splits256 > 8)
                                                      : splits256 > 16))
       split = 512;
+    // One round of workgroups: remainders of ragged lengths (or of a length
+    // just past a multiple of the split) can push the launch past one
+    // workgroup per CU, and the few that share a CU end last. The split grows
+    // until they fit, where a short split does it: 7 sequences of 200..1900
+    // tokens (32Q/8KV, 128) 16.6 -> 13.7 us per step (256 -> 320), 16 of
+    // 100..2000 21.1 -> 19.1 (576 -> 896), 32 of 50..1000 20.8 -> 17.0 (576 ->
+    // 1024). Longer splits were not measured and keep the balance above.
+    if ((int64_t)batch * kvh <= ctx->num_cus) {
+      int64_t s = split;
+      auto workgroups = [&](int64_t sp) {
+        int64_t n = 0;
+        for (int b = 0; b < batch; ++b) n += (streamed(b) + sp - 1) / sp;
+        return n * kvh;
+      };
+      while (s <= 1280 && workgroups(s) > ctx->num_cus) s += 64;
+      if (s <= 1280) split = (int32_t)s;
+    }
   }
   split = std::min(split, kMaxDecodeSplit);
   int64_t work = 0;
@@ -925,26 +942,36 @@ sai_status launch_decode(sai_ctx* ctx, sai_kvcache* c, int32_t layer, const void
   p.max_nsplit = (int)n_max;
   p.partials = ws->partials;
   p.seq_info = ws->seq_info;
-  // automatic: the last workgroup merges when every sequence has the same
-  // split count (one ticket per (sequence, kv head), measured faster at 16 x
-  // 8k, int8, and at 4 x 32k, int4); ragged batches use the combine kernel
-  // (measured faster there).
-  p.merge_in_kernel = ctx->decode_merge == 1 || (ctx->decode_merge == 2 && uniform);
+  // automatic: the last workgroup of a (sequence, kv head) merges, which saves
+  // the combine launch (16 x 8k int8, 4 x 32k int4; 7 x 200..1900: 14.6 against
+  // 16.0 us), unless there are more than 16 splits for one workgroup to read
+  // (1 x 16384, 8Q/1KV, 32 splits: 22.6 against 20.9 us) or the launch is
+  // ragged over several rounds (64 x U[128, 16384]: the combine is faster).
+  p.merge_in_kernel = ctx->decode_merge == 1 ||
+                      (ctx->decode_merge == 2 && n_max <= 16 &&
+                       (uniform || work * kvh <= 2 * ctx->num_cus));
   p.static_tiles = ctx->reproducible != 0;
   // ragged: work items go to the sequences with the longest splits first
   // (each sequence's tiles are dealt evenly to its splits, so this orders the
   // work items longest first), which the in-order dispatch of workgroups to
   // CUs then balances as a longest-processing-time list schedule
   p.ordered = 0;
-  if (!uniform && batch <= sai::kDecodeOrder) {
-    std::vector<std::pair<int64_t, int>> key((size_t)batch);
+  if (!uniform && batch <= sai::kDecodeOrder && work <= 0xFFFF) {
+    std::pair<int64_t, int> key[sai::kDecodeOrder];
     for (int b = 0; b < batch; ++b) {
       const int64_t tiles = (streamed(b) + 63) / 64;
       const int64_t n = (streamed(b) + split - 1) / split;
       key[b] = {-((tiles + n - 1) / n), b};
     }
-    std::stable_sort(key.begin(), key.end());
-    for (int i = 0; i < batch; ++i) p.order[i] = (uint16_t)key[i].second;
+    std::sort(key, key + batch);  // equal lengths in sequence order
+    int64_t end = 0;
+    for (int i = 0; i < batch; ++i) {
+      const int b = key[i].second;
+      end += (streamed(b) + split - 1) / split;
+      p.order[i] = (uint16_t)b;
+      p.item_end[i] = (uint16_t)end;
+      p.item_tps[i] = (uint16_t)-key[i].first;
+    }
     p.ordered = 1;
   }
   p.counters = ws->counters;

@@ -227,11 +227,14 @@ struct DecodeParams {
   int kv_dtype;
   int window;           // visible keys per query (0: all); see window_first_key
   int static_tiles;     // 1: fixed tile order per wave (bit-reproducible output)
-  // ragged launches (uniform_nsplit == 0) with batch <= kDecodeOrder: work
-  // items go to the sequences in this order (ordered != 0), each sequence's
-  // splits in turn
+  // ragged launches (uniform_nsplit == 0) with batch <= kDecodeOrder and at
+  // most 65535 work items (ordered != 0): the i-th sequence to be served is
+  // order[i], its splits are the work items [item_end[i - 1], item_end[i]),
+  // item_tps[i] 64-token tiles each (the last the rest)
   int ordered;
   uint16_t order[kDecodeOrder];
+  uint16_t item_end[kDecodeOrder];
+  uint16_t item_tps[kDecodeOrder];
 };
 
 struct PrefillParams {
