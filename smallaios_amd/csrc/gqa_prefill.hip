@@ -541,16 +541,30 @@ __device__ __forceinline__ void rope_q_rows(const PrefillParams& p, const int (&
 // RB row blocks of 16 attention rows per wave: 2 up to head_dim 128, 1 at
 // the stored widths 192 and 256 (the query pair and the accumulators of two
 // blocks would not fit).
+//
+// KG key groups (int8 up to head_dim 128): the waves form KG groups of NW / KG;
+// every wave stages every tile, but a group computes one tile in KG, so a
+// workgroup holds 1 / KG of the rows and passes them KG tiles at a time. The
+// groups' (m, l, o) meet in LDS at the end. For chunks whose 256-row
+// workgroups would be few (each streaming its keys one tile after the other)
+// or mostly empty; cutting their key range over workgroups instead writes
+// every row's partials to memory and merges them in another launch. KG = 4
+// takes one row block per wave (32 rows) and keeps four tiles in LDS behind a
+// second barrier: the registers of four tiles' loads need the other block's.
+// Calls at 32Q/8KV, D = 128: 1 x 1000 51.4 -> 44.1 us (KG = 2, no second launch
+// for the merge), 8 x 5 over 4000 45.8 -> 32.6 (KG = 4).
 // PREC: the int8 precise pass (see the tile loop below): only workgroups
 // whose flag the fast pass set run, from their first tile.
-template <int D, int G, int NW, int Q, bool PREC>
+template <int D, int G, int NW, int Q, bool PREC, int KG>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillParams p) {
   constexpr int NT = 64 * NW;
   constexpr int KS = D / 32;      // 32-dim k steps of QK
   constexpr int JB = D / 16;      // 16-dim column blocks of PV
-  constexpr int RB = D > 128 ? 1 : 2;
-  constexpr int QT = 16 * RB * NW / G;  // query positions per workgroup
+  constexpr int RB = D > 128 || KG == 4 ? 1 : 2;
+  constexpr int RW = NW / KG;           // waves that hold rows of their own
+  constexpr int QT = 16 * RB * RW / G;  // query positions per workgroup
   constexpr bool INT4 = Q == kQuantInt4;
+  static_assert(KG == 1 || (!INT4 && D <= 128 && KG <= 4), "key groups");
   typedef PrefillTile<D> Tile;
   constexpr int KROW = Tile::KROW;
   constexpr int VROW = Tile::VROW;
@@ -561,7 +575,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   // int4 at 256 (75 KB a tile, and the parameters) keeps one and stages behind
   // a second barrier
   constexpr int NSLOT = (!INT4 && D <= 128) ? 4 : ((INT4 && D > 128) ? 1 : 2);
-  constexpr int PER_BARRIER = NSLOT == 4 ? 2 : 1;
+  constexpr int PER_BARRIER = KG == 4 ? 4 : (NSLOT == 4 ? 2 : 1);
   __shared__ Tile sT[NSLOT];
   __shared__ Int4Params<INT4 ? D : 32> sZ[INT4 ? 3 : 1];
   // int4: each lane's query operand of the zero points' k step (registers are
@@ -571,6 +585,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
+  const int rw = __builtin_amdgcn_readfirstlane(wave % RW);  // its rows
+  const int kg = __builtin_amdgcn_readfirstlane(wave / RW);  // its tiles
   const int r = lane & 15;
   const int g = lane >> 4;
   const int kvh = blockIdx.y;
@@ -619,7 +635,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
     // a split past the rows' range: empty partials (m = -inf, l = o = 0), which
     // the merge skips
     if constexpr (!PREC) {
-      for (int e = tid; e < 16 * RB * NW * (D + 2); e += NT) {
+      for (int e = tid; e < 16 * RB * RW * (D + 2); e += NT) {
         const int R = e / (D + 2), k = e % (D + 2);
         const int il = q0 + R / G;
         if (il < p.sq) partial_of(il, R % G)[k] = k == 0 ? -INFINITY : 0.0f;
@@ -630,8 +646,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
 
   // first tile in flight while Q is prepared
   typedef typename std::conditional<INT4, TileStage4<D, NT>, TileStage<D, NT>>::type Stage;
-  Stage S;
-  StagePages<D, NT, INT4> pages;  // page ids of the next tile to load
+  constexpr int NS = KG == 4 ? 4 : 1;  // tiles whose loads are in flight at once
+  Stage Ss[NS];
+  Stage& S = Ss[0];
+  StagePages<D, NT, INT4> pgs[NS];  // page ids of the next tiles to load
+  StagePages<D, NT, INT4>& pages = pgs[0];
   StagePages<D, NT, INT4> pages2;  // int4: of the tile after it, whose parameters load with it
   auto zslot = [&](int tile) -> auto& { return sZ[INT4 ? (uint32_t)(tile - t_first) % 3u : 0]; };
   // loads tile `tile` (and the parameters of the next one), then the page ids
@@ -656,7 +675,22 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
       stage_store<D, NT>(S, slot(tile), tile * 64, total, tid);
     }
   };
-  pages.load(pt, t_first, last_page, tid);
+  // KG == 4: tiles [tile, tile + 4) at once (past the range: the last page
+  // again, staged as zero scales and never computed)
+  auto load_stage4 = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      if constexpr (!INT4) stage_load<D, NT>(Ss[i], p, pgs[i], kvh, (tile + i) * 64, tid);
+      pgs[i].load(pt, tile + NS + i, last_page, tid);
+    }
+  };
+  auto store_stage4 = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+      if constexpr (!INT4) stage_store<D, NT>(Ss[i], slot(tile + i), (tile + i) * 64, total, tid);
+  };
+#pragma unroll
+  for (int i = 0; i < NS; ++i) pgs[i].load(pt, t_first + i, last_page, tid);
   if constexpr (INT4) {
     // the first tile's parameters, and the zeros of the z rows
     pages2.load(pt, t_first + 1, last_page, tid);
@@ -666,7 +700,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
       sZ[e / (64 * (32 - NZ))].z[e / (32 - NZ) % 64 * ZR + NZ + e % (32 - NZ)] = (_Float16)0.0f;
     params_store4<D, NT>(S, zslot(t_first), t_first * 64, total, tid);
   }
-  load_stage(t_first);
+  if constexpr (KG == 4)
+    load_stage4(t_first);
+  else
+    load_stage(t_first);
 
   // ---- Q^T operand: rows R = wave*32 + rb*16 + r -> (position, head) -------
   // RoPE(q) * scale * log2(e) as an f16 pair hi + lo (~22 bits: a score's
@@ -682,7 +719,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
     size_t qrow[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      const int R = wave * (16 * RB) + rb * 16 + r;
+      const int R = rw * (16 * RB) + rb * 16 + r;
       const int il = q0 + R / G;
       const int i = il < p.sq ? il : p.sq - 1;
       pos[rb] = past + i;
@@ -756,16 +793,20 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   }
 
   if constexpr (INT4) __syncthreads();  // the first tile's parameters
-  store_stage(t_first);
-  if (PER_BARRIER == 2 && t_first + 1 < t_last) {
-    load_stage(t_first + 1);
-    store_stage(t_first + 1);
+  if constexpr (KG == 4) {
+    store_stage4(t_first);
+  } else {
+    store_stage(t_first);
+    if (PER_BARRIER == 2 && t_first + 1 < t_last) {
+      load_stage(t_first + 1);
+      store_stage(t_first + 1);
+    }
   }
   __syncthreads();
 
   // a wave whose rows all lie past the chunk only helps to stage the tiles
   const bool wave_live =
-      __builtin_amdgcn_readfirstlane(q0 + wave * (16 * RB) / G < p.sq ? 1 : 0) != 0;
+      __builtin_amdgcn_readfirstlane(q0 + rw * (16 * RB) / G < p.sq ? 1 : 0) != 0;
 
   // ---- online softmax state ----------------------------------------------------
   // m_run: the row's reference point (set from its first visible keys; 0 only
@@ -1145,6 +1186,26 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
         __syncthreads();
       }
     }
+  } else if constexpr (KG == 4) {
+    // four tiles a round, one per key group; stored once every wave has
+    // finished reading the last four
+    for (int tile = t_first; tile < t_stop; tile += 4) {
+      bool any_big = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) any_big = any_big || (tile + i < t_last && big(slot(tile + i)));
+      if (any_big) {
+        t_stop = tile;
+        break;
+      }
+      const bool more = tile + 4 < t_last;
+      if (more) load_stage4(tile + 4);
+      if (wave_live && tile + kg < t_last) process(slot(tile + kg), tile + kg);
+      __syncthreads();
+      if (more) {
+        store_stage4(tile + 4);
+        __syncthreads();
+      }
+    }
   } else {
     for (int tile = t_first; tile < t_stop; tile += PER_BARRIER) {
       // the tiles of this round are in LDS (the barrier below orders them)
@@ -1162,7 +1223,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
           const int nxt = tt + PER_BARRIER;
           const bool more = nxt < t_last;
           if (more) load_stage(nxt);
-          if (wave_live) process(slot(tt), tt);
+          if (wave_live && (KG == 1 || h == kg)) process(slot(tt), tt);
           if (more) store_stage(nxt);
         }
       }
@@ -1175,6 +1236,62 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
     return;
   }
 
+  // ---- the key groups meet (LDS is free: the loop ends behind a barrier) --------
+  if constexpr (KG > 1) {
+    constexpr int NV = RB * (4 * JB + 2) + 1;  // floats of a lane's state
+    static_assert(sizeof(float) * NV * 64 * RW * (KG - 1) <= sizeof(sT), "merge space");
+    float* sm = (float*)sT;
+    if (kg > 0) {
+      float* w = sm + (size_t)((kg - 1) * RW + rw) * NV * 64 + lane;
+      int n = 0;
+      w[64 * n++] = (float)vexp_run;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        w[64 * n++] = m_run[rb];
+        w[64 * n++] = l_run[rb];
+#pragma unroll
+        for (int jb = 0; jb < JB; ++jb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[64 * n++] = acc[rb][jb][e];
+      }
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int k = 1; k < KG; ++k) {
+      const float* w = sm + (size_t)((k - 1) * RW + rw) * NV * 64 + lane;
+      int n = 0;
+      // units of the larger exponent (precise pass; 0 otherwise)
+      const int vk = PREC ? __builtin_amdgcn_readfirstlane((int)w[0]) : 0;
+      const int vm = max(vk, vexp_run);
+      const float u0 = __builtin_ldexpf(1.0f, vexp_run - vm), uk = __builtin_ldexpf(1.0f, vk - vm);
+      vexp_run = vm;
+      ++n;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const float mk = w[64 * n++], lk = w[64 * n++];
+        // a side that has seen no key of the row weighs 0
+        const float mn = l_run[rb] > 0.0f ? (lk > 0.0f ? fmaxf(m_run[rb], mk) : m_run[rb]) : mk;
+        const float a0 = l_run[rb] > 0.0f ? fast_exp2(m_run[rb] - mn) : 0.0f;
+        const float ak = lk > 0.0f ? fast_exp2(mk - mn) : 0.0f;
+        l_run[rb] = l_run[rb] * a0 + lk * ak;
+        m_run[rb] = mn;
+        // accumulator rows 4g+e: the factors of row j live in lane j
+        float f0[4], fk[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f0[e] = __shfl(a0, 4 * g + e, 64) * u0;
+          fk[e] = __shfl(ak, 4 * g + e, 64) * uk;
+        }
+#pragma unroll
+        for (int jb = 0; jb < JB; ++jb)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[rb][jb][e] = acc[rb][jb][e] * f0[e] + w[64 * n++] * fk[e];
+      }
+    }
+  }
+
   // ---- write O / l ------------------------------------------------------------
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
@@ -1182,7 +1299,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
     for (int e = 0; e < 4; ++e) {
       const int row = 4 * g + e;  // row within the block
       const float l = __shfl(l_run[rb], row, 64);
-      const int R = wave * (16 * RB) + rb * 16 + row;
+      const int R = rw * (16 * RB) + rb * 16 + row;
       const int il = q0 + R / G;
       if (il >= p.sq) continue;
       const int hq = kvh * G + R % G;
@@ -1218,43 +1335,47 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
 // Rows per workgroup (query positions x heads of one kv head) and the grid.
 template <int D, int NW>
 dim3 prefill_grid(const PrefillParams& p, int group) {
-  constexpr int RB = D > 128 ? 1 : 2;  // as in the kernel
-  const int qt = 16 * RB * NW / group;
+  const int rb = D > 128 || p.key_groups == 4 ? 1 : 2;  // as in the kernel
+  const int qt = 16 * rb * (NW / p.key_groups) / group;
   const int nks = p.nksplit > 1 ? p.nksplit : 1;
   return dim3((p.sq + qt - 1) / qt * nks, p.kv_heads, p.batch);
 }
 
-template <int D, int NW, int Q, bool PREC>
+template <int D, int NW, int Q, bool PREC, int KG>
 hipError_t launch_pass(const PrefillParams& p, int group, hipStream_t st) {
   const dim3 grid = prefill_grid<D, NW>(p, group);
   const dim3 block(64 * NW);
   switch (group) {
-    case 1: hipLaunchKernelGGL((gqa_prefill_kernel<D, 1, NW, Q, PREC>), grid, block, 0, st, p); break;
-    case 2: hipLaunchKernelGGL((gqa_prefill_kernel<D, 2, NW, Q, PREC>), grid, block, 0, st, p); break;
-    case 4: hipLaunchKernelGGL((gqa_prefill_kernel<D, 4, NW, Q, PREC>), grid, block, 0, st, p); break;
-    case 8: hipLaunchKernelGGL((gqa_prefill_kernel<D, 8, NW, Q, PREC>), grid, block, 0, st, p); break;
+    case 1: hipLaunchKernelGGL((gqa_prefill_kernel<D, 1, NW, Q, PREC, KG>), grid, block, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((gqa_prefill_kernel<D, 2, NW, Q, PREC, KG>), grid, block, 0, st, p); break;
+    case 4: hipLaunchKernelGGL((gqa_prefill_kernel<D, 4, NW, Q, PREC, KG>), grid, block, 0, st, p); break;
+    case 8: hipLaunchKernelGGL((gqa_prefill_kernel<D, 8, NW, Q, PREC, KG>), grid, block, 0, st, p); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
 // The fast pass, then (int8) the precise pass over the workgroups it flagged.
-template <int D, int NW, int Q>
-hipError_t launch_dn(const PrefillParams& p, int group, hipStream_t st) {
-  const hipError_t e = launch_pass<D, NW, Q, false>(p, group, st);
+template <int D, int NW, int Q, int KG>
+hipError_t launch_kg(const PrefillParams& p, int group, hipStream_t st) {
+  const hipError_t e = launch_pass<D, NW, Q, false, KG>(p, group, st);
   if constexpr (Q == kQuantInt8)
-    return e != hipSuccess ? e : launch_pass<D, NW, Q, true>(p, group, st);
+    return e != hipSuccess ? e : launch_pass<D, NW, Q, true, KG>(p, group, st);
   else
     return e;
 }
 
-// 8 waves (256 rows) per workgroup: the staged K/V tile serves twice the rows
-// of a 4-wave workgroup at the same LDS footprint (measured 10% faster on the
-// 2 x 2048-over-8192 chunk).
-template <int D>
-hipError_t launch_d(const PrefillParams& p, int group, int quant, hipStream_t st) {
-  if (quant == kQuantInt4) return launch_dn<D, 8, kQuantInt4>(p, group, st);
-  return launch_dn<D, 8, kQuantInt8>(p, group, st);
+// 8 waves (256 rows with one key group) per workgroup: the staged K/V tile
+// serves twice the rows of a 4-wave workgroup at the same LDS footprint
+// (measured 10% faster on the 2 x 2048-over-8192 chunk).
+template <int D, int Q>
+hipError_t launch_d(const PrefillParams& p, int group, hipStream_t st) {
+  if constexpr (Q == kQuantInt8 && D <= 128) {
+    if (p.key_groups == 4) return launch_kg<D, 8, Q, 4>(p, group, st);
+    if (p.key_groups == 2) return launch_kg<D, 8, Q, 2>(p, group, st);
+  }
+  if (p.key_groups != 1) return hipErrorInvalidValue;
+  return launch_kg<D, 8, Q, 1>(p, group, st);
 }
 
 }  // namespace
@@ -1266,14 +1387,17 @@ size_t prefill_workgroups(const PrefillParams& p, int head_dim, int group) {
 
 hipError_t launch_gqa_prefill(const PrefillParams& p, int head_dim, int group, int quant,
                               hipStream_t st) {
-  if (quant != kQuantInt8 && quant != kQuantInt4) return hipErrorInvalidValue;
-  if (head_dim == 64) return launch_d<64>(p, group, quant, st);
-  if (head_dim == 128) return launch_d<128>(p, group, quant, st);
-  if (head_dim == 256)
-    return quant == kQuantInt8 ? launch_dn<256, 8, kQuantInt8>(p, group, st)
-                               : launch_dn<256, 8, kQuantInt4>(p, group, st);
-  // head_dim 168: the stored width 192, int8 only
-  if (head_dim == 168 && quant == kQuantInt8) return launch_dn<192, 8, kQuantInt8>(p, group, st);
+  if (quant == kQuantInt8) {
+    if (head_dim == 64) return launch_d<64, kQuantInt8>(p, group, st);
+    if (head_dim == 128) return launch_d<128, kQuantInt8>(p, group, st);
+    if (head_dim == 256) return launch_d<256, kQuantInt8>(p, group, st);
+    // head_dim 168: the stored width 192, int8 only
+    if (head_dim == 168) return launch_d<192, kQuantInt8>(p, group, st);
+  } else if (quant == kQuantInt4) {
+    if (head_dim == 64) return launch_d<64, kQuantInt4>(p, group, st);
+    if (head_dim == 128) return launch_d<128, kQuantInt4>(p, group, st);
+    if (head_dim == 256) return launch_d<256, kQuantInt4>(p, group, st);
+  }
   return hipErrorInvalidValue;
 }
 

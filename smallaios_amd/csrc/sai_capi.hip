@@ -1157,10 +1157,25 @@ SAI_API sai_status sai_gqa_prefill(sai_ctx* ctx, sai_kvcache* c, int32_t layer, 
   int64_t max_past = 0;
   for (int b = 0; b < batch; ++b) max_past = std::max<int64_t>(max_past, c->h_seq_lens[b]);
   const int64_t key_tiles = (max_past + sq + 63) / 64;
-  const int64_t base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
+  // Key groups inside the workgroup (int8, head_dim up to 128): 4 for chunks
+  // of at most 32 rows a kv head, 2 for chunks whose 256-row workgroups would
+  // be half empty or fewer than the CUs. Then the key split over workgroups
+  // for what is still short of one per CU; a split keeps at least two rounds
+  // of tiles. With two key groups a split must pay for its partials (every
+  // row's written and read again): to the nearest count, not the next.
+  p.key_groups = 1;
+  int64_t base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
+  if (c->desc.quant == SAI_KV_INT8 && D <= 128) {
+    if ((int64_t)sq * G <= 32)
+      p.key_groups = 4;
+    else if ((int64_t)sq * G <= 128 || base_wgs < 256)
+      p.key_groups = 2;
+    base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
+  }
   int nks = 1;
   if (base_wgs < 256 && key_tiles >= 16)
-    nks = (int)std::min<int64_t>((256 + base_wgs - 1) / base_wgs, key_tiles / 4);
+    nks = (int)std::min<int64_t>((256 + (p.key_groups == 2 ? base_wgs / 2 : base_wgs - 1)) / base_wgs,
+                                 key_tiles / std::max(4, 2 * p.key_groups));
   if (nks > 1) {
     p.nksplit = nks;
     p.ksplit_tiles = (int)((key_tiles + nks - 1) / nks);

@@ -258,6 +258,7 @@ struct PrefillParams {
   // one int per workgroup (prefill_workgroups), zero between launches: the
   // int8 fast pass flags the workgroups the precise pass recomputes
   int32_t* prec_flags;
+  int key_groups;  // of the waves of a workgroup (see gqa_prefill_kernel): 1, 2 or 4
   // key split (nksplit > 1): each workgroup takes ksplit_tiles 64-token tiles
   // of its rows' visible range and writes (m, l, o) partials in the decode's
   // layout (row (b, i) as sequence b * sq + i, nksplit splits each), which the

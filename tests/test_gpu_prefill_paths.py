@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 import smallaios_amd as S
-from _gpu_util import Case, assert_close, dev, err_tol_ratio, log, outlier_keys
+from _gpu_util import (Case, assert_close, assert_close_weighted, dev, err_tol_ratio, log,
+                       outlier_keys, weighted_abs_v)
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +59,47 @@ def test_prefill_int4_large_query_sums(rt, hq, hkv, d):
     ref = c.oracle_attend(q)
     log(f"  worst err/tol {err_tol_ratio(got, ref):.4f}")
     assert_close(got, ref, "prefill int4, large query sums")
+
+
+KEY_GROUPS = [
+    # hq, hkv, d, past, new, window, large V: 32, 33, 128 and 129 rows a kv
+    # head, one row, tiles that do not fill the last round of 2 or 4, rows
+    # whose first keys are another key group's
+    (8, 2, 128, [700, 0], 8, 0, False), (8, 1, 128, [300], 4, 0, False),
+    (2, 2, 64, [129, 64], 32, 0, False), (1, 1, 128, [1023], 1, 0, False),
+    (3, 3, 128, [200], 33, 0, False), (8, 2, 64, [450, 31], 32, 100, False),
+    (4, 4, 128, [5], 129, 0, False), (16, 2, 128, [63], 16, 0, False),
+    (32, 8, 128, [0], 300, 0, False), (8, 1, 64, [0, 500], 90, 70, False),
+    (8, 2, 128, [500], 8, 0, True), (8, 2, 128, [260], 60, 0, True),
+    (4, 1, 64, [1200], 7, 130, True),
+]
+
+
+@pytest.mark.parametrize("case", KEY_GROUPS, ids=[f"case{i}" for i in range(len(KEY_GROUPS))])
+def test_prefill_key_groups(rt, case):
+    """int8 chunks whose workgroups split the keys among their waves (4 key
+    groups up to 32 rows a kv head, 2 up to 128 or while workgroups are few);
+    large V takes the same split through the precise pass, bounded as in
+    test_prefill_key_split_large_v."""
+    hq, hkv, d, past, new, window, big = case
+    log(f"prefill key groups hq {hq} hkv {hkv} d {d} past {past} new {new} window {window} "
+        f"large V {big}")
+    # large V in some tokens only: the groups' tiles have different exponents
+    big_v = (lambda rng, v: v * np.where(rng.random(v.shape[:2] + (1,)) < 0.02, 1e5, 1.0)
+             .astype(np.float32)) if big else None
+    c = Case(rt, 0x9A3 + d + new, len(past), hq, hkv, d, past, new, theta=5e5,
+             permute_pages=True, k_transform=outlier_keys(d, (3, 40)) if not big else None,
+             v_transform=big_v)
+    c.step_kv()
+    q = c.query("f32")
+    got = c.gpu_prefill(q, "f32", window=window)
+    ref = c.oracle_attend(q, mask_window=window)
+    if big and window == 0:
+        assert np.isfinite(got).all()
+        assert_close_weighted(got, ref, weighted_abs_v(c, q), 2.0 ** -12, "key groups, large V")
+    elif big:
+        # Sum p|v| of the window is at most the rows' largest |v| there
+        assert (np.abs(got - ref) <= 2e-3 + 1e-2 * np.abs(ref) + 2.0 ** -12 * 6e5).all()
+    else:
+        log(f"  worst err/tol {err_tol_ratio(got, ref):.4f}")
+        assert_close(got, ref, "prefill key groups")
