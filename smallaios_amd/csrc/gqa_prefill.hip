@@ -265,6 +265,12 @@ __device__ __forceinline__ void stage_store(const TileStage<D, NT>& S, Tile& T, 
   }
 }
 
+// Key groups a workgroup can form (see gqa_prefill_kernel): as many as tiles
+// fit the LDS at once. Above head_dim 128 one: two int8 tiles fit, but their
+// loads do not fit the registers beside the query (56 to 103 spilled).
+template <int D, int Q>
+constexpr int kMaxKeyGroups = D > 128 ? 1 : (Q == kQuantInt4 ? 2 : 4);
+
 // ---- int4 cache ---------------------------------------------------------------
 // K = code * s + z with (s, z) per token and group of 32 dims, and a group is
 // exactly one k step of the QK product. So the K tile holds the bare codes,
@@ -542,15 +548,17 @@ __device__ __forceinline__ void rope_q_rows(const PrefillParams& p, const int (&
 // the stored widths 192 and 256 (the query pair and the accumulators of two
 // blocks would not fit).
 //
-// KG key groups (int8 up to head_dim 128): the waves form KG groups of NW / KG;
-// every wave stages every tile, but a group computes one tile in KG, so a
-// workgroup holds 1 / KG of the rows and passes them KG tiles at a time. The
+// KG key groups: the waves form KG groups of NW / KG; every wave stages every
+// tile, but a group computes one tile in KG, so a workgroup holds 1 / KG of
+// the rows and passes them KG tiles at a time. The
 // groups' (m, l, o) meet in LDS at the end. For chunks whose 256-row
 // workgroups would be few (each streaming its keys one tile after the other)
 // or mostly empty; cutting their key range over workgroups instead writes
-// every row's partials to memory and merges them in another launch. KG = 4
-// takes one row block per wave (32 rows) and keeps four tiles in LDS behind a
-// second barrier: the registers of four tiles' loads need the other block's.
+// every row's partials to memory and merges them in another launch. KG = 2
+// uses the four tile slots of int8 as one group does; int4 has LDS for a round
+// only, stored behind a second barrier, and so has KG = 4 (int8), which takes
+// one row block per wave (32 rows): the registers of four tiles' loads need
+// the other block's.
 // Calls at 32Q/8KV, D = 128: 1 x 1000 51.4 -> 44.1 us (KG = 2, no second launch
 // for the merge), 8 x 5 over 4000 45.8 -> 32.6 (KG = 4).
 // PREC: the int8 precise pass (see the tile loop below): only workgroups
@@ -564,7 +572,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   constexpr int RW = NW / KG;           // waves that hold rows of their own
   constexpr int QT = 16 * RB * RW / G;  // query positions per workgroup
   constexpr bool INT4 = Q == kQuantInt4;
-  static_assert(KG == 1 || (!INT4 && D <= 128 && KG <= 4), "key groups");
+  static_assert(KG <= kMaxKeyGroups<D, Q>, "key groups");
+  // rounds of KG tiles whose loads wait in registers for the round's end
+  constexpr bool ROUNDS = KG == 4 || (KG == 2 && INT4);
   typedef PrefillTile<D> Tile;
   constexpr int KROW = Tile::KROW;
   constexpr int VROW = Tile::VROW;
@@ -575,9 +585,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   // int4 at 256 (75 KB a tile, and the parameters) keeps one and stages behind
   // a second barrier
   constexpr int NSLOT = (!INT4 && D <= 128) ? 4 : ((INT4 && D > 128) ? 1 : 2);
-  constexpr int PER_BARRIER = KG == 4 ? 4 : (NSLOT == 4 ? 2 : 1);
+  constexpr int PER_BARRIER = ROUNDS ? KG : (NSLOT == 4 ? 2 : 1);
+  // tiles whose int4 parameters are held: those computed, those staged next
+  // and (one barrier) the ones after
+  constexpr int ZN = ROUNDS ? 2 * KG : 3;
   __shared__ Tile sT[NSLOT];
-  __shared__ Int4Params<INT4 ? D : 32> sZ[INT4 ? 3 : 1];
+  __shared__ Int4Params<INT4 ? D : 32> sZ[INT4 ? ZN : 1];
   // int4: each lane's query operand of the zero points' k step (registers are
   // what this kernel is short of; a lane reads back its own)
   __shared__ v8h sQZ[INT4 ? NW * RB : 1][64];
@@ -646,64 +659,59 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
 
   // first tile in flight while Q is prepared
   typedef typename std::conditional<INT4, TileStage4<D, NT>, TileStage<D, NT>>::type Stage;
-  constexpr int NS = KG == 4 ? 4 : 1;  // tiles whose loads are in flight at once
+  constexpr int NS = ROUNDS ? KG : 1;  // tiles whose loads are in flight at once
   Stage Ss[NS];
-  Stage& S = Ss[0];
-  StagePages<D, NT, INT4> pgs[NS];  // page ids of the next tiles to load
-  StagePages<D, NT, INT4>& pages = pgs[0];
-  StagePages<D, NT, INT4> pages2;  // int4: of the tile after it, whose parameters load with it
-  auto zslot = [&](int tile) -> auto& { return sZ[INT4 ? (uint32_t)(tile - t_first) % 3u : 0]; };
-  // loads tile `tile` (and the parameters of the next one), then the page ids
-  // of the tiles after
-  auto load_stage = [&](int tile) {
-    if constexpr (INT4) {
-      stage_load4<D, NT>(S, p, pages, kvh, tid);
-      params_load4<D, NT>(S, p, pages2, kvh, tid);
-      pages = pages2;
-      pages2.load(pt, tile + 2, last_page, tid);
-    } else {
-      stage_load<D, NT>(S, p, pages, kvh, tile * 64, tid);
-      pages.load(pt, tile + 1, last_page, tid);
-    }
-  };
+  StagePages<D, NT, INT4> pages[NS];  // page ids of the next tiles to load
+  // int4: of the tiles after them, whose parameters load with them
+  StagePages<D, NT, INT4> pages2[NS];
+  auto zslot = [&](int tile) -> auto& { return sZ[INT4 ? (uint32_t)(tile - t_first) % ZN : 0]; };
   auto slot = [&](int tile) -> Tile& { return sT[(tile - t_first) & (NSLOT - 1)]; };
-  auto store_stage = [&](int tile) {
-    if constexpr (INT4) {
-      params_store4<D, NT>(S, zslot(tile + 1), (tile + 1) * 64, total, tid);
-      stage_store4<D, NT>(S, slot(tile), zslot(tile), tid);
-    } else {
-      stage_store<D, NT>(S, slot(tile), tile * 64, total, tid);
-    }
-  };
-  // KG == 4: tiles [tile, tile + 4) at once (past the range: the last page
-  // again, staged as zero scales and never computed)
-  auto load_stage4 = [&](int tile) {
+  // loads tiles [tile, tile + NS) (and the parameters of the NS after), then
+  // the page ids of the tiles after. Tiles past the range read its last page;
+  // they are staged as zero scales and never computed.
+  auto load_stage = [&](int tile) {
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-      if constexpr (!INT4) stage_load<D, NT>(Ss[i], p, pgs[i], kvh, (tile + i) * 64, tid);
-      pgs[i].load(pt, tile + NS + i, last_page, tid);
+      if constexpr (INT4) {
+        stage_load4<D, NT>(Ss[i], p, pages[i], kvh, tid);
+        params_load4<D, NT>(Ss[i], p, pages2[i], kvh, tid);
+        pages[i] = pages2[i];
+        pages2[i].load(pt, tile + 2 * NS + i, last_page, tid);
+      } else {
+        stage_load<D, NT>(Ss[i], p, pages[i], kvh, (tile + i) * 64, tid);
+        pages[i].load(pt, tile + NS + i, last_page, tid);
+      }
     }
   };
-  auto store_stage4 = [&](int tile) {
+  auto store_stage = [&](int tile) {
 #pragma unroll
-    for (int i = 0; i < NS; ++i)
-      if constexpr (!INT4) stage_store<D, NT>(Ss[i], slot(tile + i), (tile + i) * 64, total, tid);
+    for (int i = 0; i < NS; ++i) {
+      const int t = tile + i;
+      if constexpr (INT4) {
+        params_store4<D, NT>(Ss[i], zslot(t + NS), (t + NS) * 64, total, tid);
+        stage_store4<D, NT>(Ss[i], slot(t), zslot(t), tid);
+      } else {
+        stage_store<D, NT>(Ss[i], slot(t), t * 64, total, tid);
+      }
+    }
   };
 #pragma unroll
-  for (int i = 0; i < NS; ++i) pgs[i].load(pt, t_first + i, last_page, tid);
+  for (int i = 0; i < NS; ++i) pages[i].load(pt, t_first + i, last_page, tid);
   if constexpr (INT4) {
-    // the first tile's parameters, and the zeros of the z rows
-    pages2.load(pt, t_first + 1, last_page, tid);
-    params_load4<D, NT>(S, p, pages, kvh, tid);
+    // the first tiles' parameters, and the zeros of the z rows
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      pages2[i].load(pt, t_first + NS + i, last_page, tid);
+      params_load4<D, NT>(Ss[i], p, pages[i], kvh, tid);
+    }
     constexpr int ZR = Int4Params<D>::ZROW, NZ = 2 * (D / 32);
-    for (int e = tid; e < 3 * 64 * (32 - NZ); e += NT)
+    for (int e = tid; e < ZN * 64 * (32 - NZ); e += NT)
       sZ[e / (64 * (32 - NZ))].z[e / (32 - NZ) % 64 * ZR + NZ + e % (32 - NZ)] = (_Float16)0.0f;
-    params_store4<D, NT>(S, zslot(t_first), t_first * 64, total, tid);
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+      params_store4<D, NT>(Ss[i], zslot(t_first + i), (t_first + i) * 64, total, tid);
   }
-  if constexpr (KG == 4)
-    load_stage4(t_first);
-  else
-    load_stage(t_first);
+  load_stage(t_first);
 
   // ---- Q^T operand: rows R = wave*32 + rb*16 + r -> (position, head) -------
   // RoPE(q) * scale * log2(e) as an f16 pair hi + lo (~22 bits: a score's
@@ -793,14 +801,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   }
 
   if constexpr (INT4) __syncthreads();  // the first tile's parameters
-  if constexpr (KG == 4) {
-    store_stage4(t_first);
-  } else {
-    store_stage(t_first);
-    if (PER_BARRIER == 2 && t_first + 1 < t_last) {
-      load_stage(t_first + 1);
-      store_stage(t_first + 1);
-    }
+  store_stage(t_first);
+  if (!ROUNDS && PER_BARRIER == 2 && t_first + 1 < t_last) {
+    load_stage(t_first + 1);
+    store_stage(t_first + 1);
   }
   __syncthreads();
 
@@ -1186,23 +1190,23 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
         __syncthreads();
       }
     }
-  } else if constexpr (KG == 4) {
-    // four tiles a round, one per key group; stored once every wave has
-    // finished reading the last four
-    for (int tile = t_first; tile < t_stop; tile += 4) {
+  } else if constexpr (ROUNDS) {
+    // KG tiles a round, one per key group; the next ones stored once every
+    // wave has finished reading these
+    for (int tile = t_first; tile < t_stop; tile += KG) {
       bool any_big = false;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) any_big = any_big || (tile + i < t_last && big(slot(tile + i)));
+      for (int i = 0; i < KG; ++i) any_big = any_big || (tile + i < t_last && big(slot(tile + i)));
       if (any_big) {
         t_stop = tile;
         break;
       }
-      const bool more = tile + 4 < t_last;
-      if (more) load_stage4(tile + 4);
+      const bool more = tile + KG < t_last;
+      if (more) load_stage(tile + KG);
       if (wave_live && tile + kg < t_last) process(slot(tile + kg), tile + kg);
       __syncthreads();
       if (more) {
-        store_stage4(tile + 4);
+        store_stage(tile + KG);
         __syncthreads();
       }
     }
@@ -1370,10 +1374,10 @@ hipError_t launch_kg(const PrefillParams& p, int group, hipStream_t st) {
 // (measured 10% faster on the 2 x 2048-over-8192 chunk).
 template <int D, int Q>
 hipError_t launch_d(const PrefillParams& p, int group, hipStream_t st) {
-  if constexpr (Q == kQuantInt8 && D <= 128) {
+  if constexpr (kMaxKeyGroups<D, Q> >= 4)
     if (p.key_groups == 4) return launch_kg<D, 8, Q, 4>(p, group, st);
+  if constexpr (kMaxKeyGroups<D, Q> >= 2)
     if (p.key_groups == 2) return launch_kg<D, 8, Q, 2>(p, group, st);
-  }
   if (p.key_groups != 1) return hipErrorInvalidValue;
   return launch_kg<D, 8, Q, 1>(p, group, st);
 }
@@ -1383,6 +1387,11 @@ hipError_t launch_d(const PrefillParams& p, int group, hipStream_t st) {
 size_t prefill_workgroups(const PrefillParams& p, int head_dim, int group) {
   const dim3 g = head_dim > 128 ? prefill_grid<256, 8>(p, group) : prefill_grid<128, 8>(p, group);
   return (size_t)g.x * g.y * g.z;
+}
+
+int prefill_max_key_groups(int head_dim, int quant) {
+  if (quant == kQuantInt4) return head_dim <= 128 ? kMaxKeyGroups<128, kQuantInt4> : kMaxKeyGroups<256, kQuantInt4>;
+  return head_dim <= 128 ? kMaxKeyGroups<128, kQuantInt8> : kMaxKeyGroups<256, kQuantInt8>;
 }
 
 hipError_t launch_gqa_prefill(const PrefillParams& p, int head_dim, int group, int quant,

@@ -1157,21 +1157,32 @@ SAI_API sai_status sai_gqa_prefill(sai_ctx* ctx, sai_kvcache* c, int32_t layer, 
   int64_t max_past = 0;
   for (int b = 0; b < batch; ++b) max_past = std::max<int64_t>(max_past, c->h_seq_lens[b]);
   const int64_t key_tiles = (max_past + sq + 63) / 64;
-  // Key groups inside the workgroup (int8, head_dim up to 128): 4 for chunks
-  // of at most 32 rows a kv head, 2 for chunks whose 256-row workgroups would
-  // be half empty or fewer than the CUs. Then the key split over workgroups
-  // for what is still short of one per CU; a split keeps at least two rounds
-  // of tiles. With two key groups a split must pay for its partials (every
-  // row's written and read again): to the nearest count, not the next.
+  // Key groups inside the workgroup (head_dim up to 128; us per call at
+  // 32Q/8KV, D = 128, 1 group / 2 / 4):
+  //   4 (int8) for chunks of at most 32 rows a kv head: 16 x 8 over 4000
+  //     85.8 / 70.2 / 51.7, 1 x 16 over 8192 29.9 / 28.9 / 27.5;
+  //   2 for at most 128 rows a kv head, where 256-row workgroups are half
+  //     empty: 16 x 32 over 4000 100.2 / 81.5 (int4 111.7 / 97.4);
+  //   2 where 128-row workgroups still fit the CUs once: 1 x 1000 51.4 / 42.6,
+  //     1 x 1024 over 3000 124.5 / 113.8; int8 also where they do not but the
+  //     key split below would cut the 256-row ones; 4 x 400 (224 workgroups
+  //     of 256 rows, no split) is 35.5 / 47.6. int4 pays a second barrier a
+  //     round: 1 x 1000 60.2 / 55.2, but 1 x 1024 over 3000 149.3 / 154.9.
+  // Then the key split over workgroups for what is still short of one per CU;
+  // a split keeps at least two rounds of tiles. With two key groups a split
+  // must pay for its partials (every row's written and read again): to the
+  // nearest count, not the next.
   p.key_groups = 1;
   int64_t base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
-  if (c->desc.quant == SAI_KV_INT8 && D <= 128) {
-    if ((int64_t)sq * G <= 32)
-      p.key_groups = 4;
-    else if ((int64_t)sq * G <= 128 || base_wgs < 256)
-      p.key_groups = 2;
-    base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
-  }
+  const int max_groups = sai::prefill_max_key_groups(D, c->desc.quant);
+  const bool few = c->desc.quant == SAI_KV_INT8
+                       ? base_wgs <= 128 || (base_wgs < 256 && key_tiles >= 16)
+                       : base_wgs <= 128 && key_tiles <= 32;
+  if (max_groups >= 4 && (int64_t)sq * G <= 32)
+    p.key_groups = 4;
+  else if (max_groups >= 2 && ((int64_t)sq * G <= 128 || few))
+    p.key_groups = 2;
+  base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
   int nks = 1;
   if (base_wgs < 256 && key_tiles >= 16)
     nks = (int)std::min<int64_t>((256 + (p.key_groups == 2 ? base_wgs / 2 : base_wgs - 1)) / base_wgs,

@@ -81,13 +81,26 @@ def test_prefill_key_groups(rt, case):
     groups up to 32 rows a kv head, 2 up to 128 or while workgroups are few);
     large V takes the same split through the precise pass, bounded as in
     test_prefill_key_split_large_v."""
-    hq, hkv, d, past, new, window, big = case
-    log(f"prefill key groups hq {hq} hkv {hkv} d {d} past {past} new {new} window {window} "
+    key_groups_case(rt, S.KV_INT8, *case)
+
+
+@pytest.mark.parametrize("case", [
+    (8, 2, 128, [700, 0], 8, 0, False), (2, 2, 64, [129, 64], 128, 0, False),
+    (1, 1, 128, [1023], 1, 0, False), (3, 3, 64, [200], 33, 100, False),
+    (32, 8, 128, [0], 300, 0, False), (8, 1, 128, [400, 70], 90, 70, False)],
+    ids=[f"case{i}" for i in range(6)])
+def test_prefill_key_groups_int4(rt, case):
+    """Two key groups over the int4 cache (its parameters in a ring of four)."""
+    key_groups_case(rt, S.KV_INT4, *case)
+
+
+def key_groups_case(rt, quant, hq, hkv, d, past, new, window, big):
+    log(f"prefill key groups quant {quant} hq {hq} hkv {hkv} d {d} past {past} new {new} window {window} "
         f"large V {big}")
     # large V in some tokens only: the groups' tiles have different exponents
     big_v = (lambda rng, v: v * np.where(rng.random(v.shape[:2] + (1,)) < 0.02, 1e5, 1.0)
              .astype(np.float32)) if big else None
-    c = Case(rt, 0x9A3 + d + new, len(past), hq, hkv, d, past, new, theta=5e5,
+    c = Case(rt, 0x9A3 + d + new, len(past), hq, hkv, d, past, new, theta=5e5, quant=quant,
              permute_pages=True, k_transform=outlier_keys(d, (3, 40)) if not big else None,
              v_transform=big_v)
     c.step_kv()
