@@ -41,7 +41,7 @@
 // flight while tile i is computed).
 //
 // Work split: grid.x enumerates (sequence, split) pairs over ragged lengths
-// (each wave finds its pair by a prefix scan over seq_lens), grid.y is the kv
+// (from the host's table or a prefix scan over seq_lens), grid.y is the kv
 // head. The NW waves of a workgroup take the split's tiles from an LDS
 // counter and merge through LDS. A sequence with one split writes its output
 // directly; with several, every workgroup writes a partial (m, l, o), and

@@ -117,16 +117,14 @@ __device__ __forceinline__ float load_row_elem(const void* p, size_t i, bool bf1
 }
 
 // One butterfly stage below 64: dims l and l ^ H of each lane pair into
-// (a + b, a - b), the sum at the lower dim: the partner plus or minus the
-// lane's own value, the sign as an exact product (no select of two sums).
+// (a + b, a - b), the sum at the lower dim.
 template <int H, int E>
 __device__ __forceinline__ void butterfly_stage(float (&y)[E], int lane) {
 #pragma clang fp contract(off)
-  const float own = (lane & H) ? -1.0f : 1.0f;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const float p = lane_xor<H>(y[e], lane);
-    y[e] = y[e] * own + p;
+    y[e] = (lane & H) ? p - y[e] : y[e] + p;
   }
 }
 
@@ -333,6 +331,17 @@ __device__ __forceinline__ void wave_store_row(const TqArgs& a, const float (&x)
 // those chains 64 times over per tile: a 2 x 1024-row pass (8 kv heads, D =
 // 128, 4 bits, QJL, bf16; 23 MB, 3 us at 8 TB/s) took 133 us and takes 14.1 (19
 // with an IEEE division for every code).
+//
+// A stage across lanes: the partner plus or minus the lane's own value, the
+// sign as an exact product (no select of two sums; the attention kernel's
+// register budget is better off with the select).
+template <int H>
+__device__ __forceinline__ void lane32_stage(float (&y)[32], int lane) {
+#pragma clang fp contract(off)
+  const float own = (lane & H) ? -1.0f : 1.0f;
+#pragma unroll
+  for (int e = 0; e < 32; ++e) y[e] = y[e] * own + lane_xor<H>(y[e], lane);
+}
 template <int D>
 __device__ __forceinline__ void lane32_butterfly(float (&y)[32], int lane, float norm) {
 #pragma clang fp contract(off)
@@ -345,9 +354,9 @@ __device__ __forceinline__ void lane32_butterfly(float (&y)[32], int lane, float
         y[e] = a0 + a1;
         y[e + hs] = a0 - a1;
       }
-  butterfly_stage<1>(y, lane);  // dims 32 apart: neighbouring lanes
-  if constexpr (D >= 128) butterfly_stage<2>(y, lane);
-  if constexpr (D >= 256) butterfly_stage<4>(y, lane);
+  lane32_stage<1>(y, lane);  // dims 32 apart: neighbouring lanes
+  if constexpr (D >= 128) lane32_stage<2>(y, lane);
+  if constexpr (D >= 256) lane32_stage<4>(y, lane);
 #pragma unroll
   for (int e = 0; e < 32; ++e) y[e] *= norm;
 }
