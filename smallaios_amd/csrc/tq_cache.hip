@@ -456,10 +456,10 @@ __global__ __launch_bounds__(2 * D) void tq_write_kernel(const TqArgs a, const v
     uint32_t cb[8] = {};  // the lane's codes, a byte each
     float csum = 0.0f;    // integers below 2^24: exact
     if (__ballot(!(range < INFINITY && scale >= 1e-30f)) == 0) {
-      // Finite rows: the quotient t = (y - zero) / scale >= 0 as a product with
-      // the scale's reciprocal. That is within 2^-22 t of the rounded
-      // quotient, so away from the half-integers both round to the same code;
-      // within NEAR of one, the quotient itself decides.
+      // Rows of finite range: the quotient t = (y - zero) / scale >= 0 as a
+      // product with the scale's reciprocal. That is within 2^-22 t of the
+      // rounded quotient, so away from the half-integers both round to the same
+      // code; within NEAR of one, the quotient itself decides.
       constexpr float NEAR = (float)LEVELS / (float)(1 << 20);
       const float rs = __builtin_amdgcn_rcpf(scale);
 #pragma unroll
@@ -468,7 +468,9 @@ __global__ __launch_bounds__(2 * D) void tq_write_kernel(const TqArgs a, const v
         float cf = __builtin_rintf(t);
         if (__ballot(fabsf(__builtin_amdgcn_fractf(t) - 0.5f) <= NEAR) != 0)
           cf = round_half_away(d / scale);
-        cf = fminf(cf, (float)LEVELS);
+        // 0..LEVELS; a NaN (rows that overflowed in part: the minimum and the
+        // maximum skip it) gives the smallest operand, code 0
+        cf = __builtin_amdgcn_fmed3f(cf, 0.0f, (float)LEVELS);
         cb[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(cf, e & 3, cb[e >> 2]);
         csum += cf;
         y[e] = cf * scale + zero;

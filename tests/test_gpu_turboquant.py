@@ -197,6 +197,47 @@ def test_write_rows_at_tile_edges(rt, d, bits, bf16, shift):
         c.close()
 
 
+@pytest.mark.parametrize("d,bits", [(64, 3), (64, 8), (128, 4), (128, 8), (256, 3), (256, 4)])
+def test_write_partly_overflowed_rows(rt, d, bits):
+    """Rows whose butterfly overflows with both signs: NaN in some rotated
+    dims, finite values (and no infinity) in the others. The minimum and the
+    maximum skip NaN, so such a row has a finite range like its neighbours; a
+    NaN element's code is 0. Codes, scale and zero point bit for bit (the
+    decoded rows hold NaN, whose sign is not pinned)."""
+    import torch
+    log(f"tq write, partly overflowed rows d={d} bits={bits}")
+    rng = np.random.default_rng(d + bits)
+    batch, heads, n = 1, 2, 70
+    # signs of eight rotated-domain entries of 3e38 that leave NaN and finite
+    # dims only
+    masks = [3, 12, 48, 63, 86, 89]
+    sg = [head_signs(SEED, 0, heads, h, d).astype(np.float32) for h in range(heads)]
+    xs = []
+    for _ in range(2):
+        x = rng.standard_normal((batch, n, heads, d)).astype(np.float32)
+        for i in range(0, n, 5):
+            m = masks[i // 5 % len(masks)]
+            for h in range(heads):
+                x[0, i, h, :8] = np.where([(m >> j) & 1 for j in range(8)], -3e38, 3e38)
+                x[0, i, h] *= sg[h]
+        xs.append(x.reshape(batch, n, heads * d))
+    c = S.TqCache(rt, 1, heads, d, bits, False, batch, n, seed=SEED)
+    try:
+        c.write(0, to_dev(xs[0], False), to_dev(xs[1], False), batch, n)
+        c.advance()
+        torch.cuda.synchronize()
+        for h in range(heads):
+            raw = c.read_raw(0, 0, h, 0, n)
+            for kind, x in (("k", xs[0]), ("v", xs[1])):
+                codes, sc, z, _, _ = O.tq_write_rows(rows_of(x, 0, h, heads, d), bits, sg[h], False)
+                assert np.isfinite(sc).all() and np.isfinite(z).all()
+                assert np.array_equal(raw[f"{kind}_codes"], codes), (kind, h)
+                assert np.array_equal(raw[f"{kind}_params"][:, 0].view(np.uint32), sc.view(np.uint32))
+                assert np.array_equal(raw[f"{kind}_params"][:, 1].view(np.uint32), z.view(np.uint32))
+    finally:
+        c.close()
+
+
 def test_constant_and_edge_rows(rt):
     """Constant rows (range 0: scale 1.0), zeros, large magnitudes."""
     import torch
