@@ -182,42 +182,59 @@ def _dev_ptr(x):
     return x.data_ptr()
 
 
-_torch_state = None  # (torch, its dtypes' codes), or (None, {}) without torch
+_torch_state = None  # what _torch() returns
 
 
 def _torch():
+    """(torch, its dtypes' codes, a function that gives its current stream's
+    handle); torch None where it is not installed."""
     global _torch_state
     if _torch_state is None:
         try:
             import torch
             _torch_state = (torch, {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16,
-                                    torch.float16: DTYPE_F16})
+                                    torch.float16: DTYPE_F16}, _current_stream_of(torch))
         except ImportError:  # pragma: no cover
-            _torch_state = (None, {})
+            _torch_state = (None, {}, lambda: None)
     return _torch_state
 
 
+def _current_stream_of(torch):
+    """A function that gives the hipStream_t of torch's current stream.
+
+    It reads the handle as a number: building the Stream object that
+    torch.cuda.current_stream() returns took 2.9 of the 9.9 us a decode call
+    took on the host (the smallest step's kernel takes 7.3). torch keeps the
+    two functions for that private, so the public call serves where one of them
+    is missing, and before torch has initialised the GPU."""
+    def public():
+        try:
+            return torch.cuda.current_stream().cuda_stream
+        except Exception:
+            # only a torch without a GPU has no current stream: any other
+            # failure must not end in an unordered launch on the null stream
+            if torch.cuda.is_available():
+                raise
+            return None
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    if raw is None or device is None:
+        return public
+    return lambda: raw(device()) if torch.cuda.is_initialized() else public()
+
+
 def _dtype_code(x, default=DTYPE_F32):
-    torch, codes = _torch()
+    torch, codes, _ = _torch()
     if torch is not None and isinstance(x, torch.Tensor):
         return codes[x.dtype]
     return default
 
 
 def _stream(stream):
-    """The hipStream_t of `stream`, or of torch's current stream.
-
-    The current stream's handle is read as a number: building the Stream
-    object that torch.cuda.current_stream() returns took 2.9 of the 9.9 us a
-    decode call took on the host (the smallest step's kernel takes 7.3)."""
+    """The hipStream_t of `stream`, or of torch's current stream."""
     if stream is None:
-        torch, _ = _torch()
-        try:
-            if torch.cuda.is_initialized():
-                return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
-            return torch.cuda.current_stream().cuda_stream
-        except Exception:  # pragma: no cover
-            return None
+        return _torch()[2]()
     return stream if isinstance(stream, int) else stream.cuda_stream
 
 
