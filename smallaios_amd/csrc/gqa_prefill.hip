@@ -28,6 +28,7 @@
 // key of a sliding window, apply the mask.
 #include <type_traits>
 
+#include "prefill_plan.h"
 #include "sai_internal.h"
 
 namespace sai {
@@ -264,12 +265,6 @@ __device__ __forceinline__ void stage_store(const TileStage<D, NT>& S, Tile& T, 
     }
   }
 }
-
-// Key groups a workgroup can form (see gqa_prefill_kernel): as many as tiles
-// fit the LDS at once. Above head_dim 128 one: two int8 tiles fit, but their
-// loads do not fit the registers beside the query (56 to 103 spilled).
-template <int D, int Q>
-constexpr int kMaxKeyGroups = D > 128 ? 1 : (Q == kQuantInt4 ? 2 : 4);
 
 // ---- int4 cache ---------------------------------------------------------------
 // K = code * s + z with (s, z) per token and group of 32 dims, and a group is
@@ -568,11 +563,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   constexpr int NT = 64 * NW;
   constexpr int KS = D / 32;      // 32-dim k steps of QK
   constexpr int JB = D / 16;      // 16-dim column blocks of PV
-  constexpr int RB = D > 128 || KG == 4 ? 1 : 2;
+  constexpr int RB = prefill_row_blocks(D, KG);
   constexpr int RW = NW / KG;           // waves that hold rows of their own
   constexpr int QT = 16 * RB * RW / G;  // query positions per workgroup
   constexpr bool INT4 = Q == kQuantInt4;
-  static_assert(KG <= kMaxKeyGroups<D, Q>, "key groups");
+  static_assert(KG <= prefill_max_key_groups(D, INT4), "key groups");
   // rounds of KG tiles whose loads wait in registers for the round's end
   constexpr bool ROUNDS = KG == 4 || (KG == 2 && INT4);
   typedef PrefillTile<D> Tile;
@@ -1336,18 +1331,17 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   }
 }
 
-// Rows per workgroup (query positions x heads of one kv head) and the grid.
-template <int D, int NW>
-dim3 prefill_grid(const PrefillParams& p, int group) {
-  const int rb = D > 128 || p.key_groups == 4 ? 1 : 2;  // as in the kernel
-  const int qt = 16 * rb * (NW / p.key_groups) / group;
+// The grid: (row blocks x key splits, kv heads, sequences).
+dim3 prefill_grid(const PrefillParams& p, int head_dim, int group) {
+  const int qt = prefill_workgroup_rows(head_dim, p.key_groups) / group;
   const int nks = p.nksplit > 1 ? p.nksplit : 1;
   return dim3((p.sq + qt - 1) / qt * nks, p.kv_heads, p.batch);
 }
 
 template <int D, int NW, int Q, bool PREC, int KG>
 hipError_t launch_pass(const PrefillParams& p, int group, hipStream_t st) {
-  const dim3 grid = prefill_grid<D, NW>(p, group);
+  static_assert(NW == 8, "prefill_workgroup_rows");
+  const dim3 grid = prefill_grid(p, D, group);
   const dim3 block(64 * NW);
   switch (group) {
     case 1: hipLaunchKernelGGL((gqa_prefill_kernel<D, 1, NW, Q, PREC, KG>), grid, block, 0, st, p); break;
@@ -1374,9 +1368,9 @@ hipError_t launch_kg(const PrefillParams& p, int group, hipStream_t st) {
 // (measured 10% faster on the 2 x 2048-over-8192 chunk).
 template <int D, int Q>
 hipError_t launch_d(const PrefillParams& p, int group, hipStream_t st) {
-  if constexpr (kMaxKeyGroups<D, Q> >= 4)
+  if constexpr (prefill_max_key_groups(D, Q == kQuantInt4) >= 4)
     if (p.key_groups == 4) return launch_kg<D, 8, Q, 4>(p, group, st);
-  if constexpr (kMaxKeyGroups<D, Q> >= 2)
+  if constexpr (prefill_max_key_groups(D, Q == kQuantInt4) >= 2)
     if (p.key_groups == 2) return launch_kg<D, 8, Q, 2>(p, group, st);
   if (p.key_groups != 1) return hipErrorInvalidValue;
   return launch_kg<D, 8, Q, 1>(p, group, st);
@@ -1385,13 +1379,8 @@ hipError_t launch_d(const PrefillParams& p, int group, hipStream_t st) {
 }  // namespace
 
 size_t prefill_workgroups(const PrefillParams& p, int head_dim, int group) {
-  const dim3 g = head_dim > 128 ? prefill_grid<256, 8>(p, group) : prefill_grid<128, 8>(p, group);
+  const dim3 g = prefill_grid(p, head_dim, group);
   return (size_t)g.x * g.y * g.z;
-}
-
-int prefill_max_key_groups(int head_dim, int quant) {
-  if (quant == kQuantInt4) return head_dim <= 128 ? kMaxKeyGroups<128, kQuantInt4> : kMaxKeyGroups<256, kQuantInt4>;
-  return head_dim <= 128 ? kMaxKeyGroups<128, kQuantInt8> : kMaxKeyGroups<256, kQuantInt8>;
 }
 
 hipError_t launch_gqa_prefill(const PrefillParams& p, int head_dim, int group, int quant,

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/sai_hip.h"
+#include "prefill_plan.h"
 #include "sai_internal.h"
 
 #define SAI_API extern "C" __attribute__((visibility("default")))
@@ -1147,49 +1148,25 @@ SAI_API sai_status sai_gqa_prefill(sai_ctx* ctx, sai_kvcache* c, int32_t layer, 
   const float sc = has_scale ? scale : sai_default_scale(D);
   p.scale_log2 = sc * 1.4426950408889634f;
   p.window = visible_span(c->layer_window[layer], window);
-  // Key split: a short chunk over a long past has few workgroups (one per
-  // 256 rows and kv head), each streaming the whole visible past. With fewer
-  // than 256 of them (one per CU) and at least 16 tiles to stream, the rows'
-  // key range is cut into splits of at least 4 tiles, to about 256
-  // workgroups, and the decode's combine kernel merges the partials (each row
-  // of the chunk a sequence of its own). 1 x 8192 past, 32Q/8KV: 16 tokens
-  // 334 -> 35 us, 1024 tokens 381 -> 228 us (the c5 chunk has 512 workgroups).
-  int64_t max_past = 0;
-  for (int b = 0; b < batch; ++b) max_past = std::max<int64_t>(max_past, c->h_seq_lens[b]);
-  const int64_t key_tiles = (max_past + sq + 63) / 64;
-  // Key groups inside the workgroup (head_dim up to 128; us per call at
-  // 32Q/8KV, D = 128, 1 group / 2 / 4):
-  //   4 (int8) for chunks of at most 32 rows a kv head: 16 x 8 over 4000
-  //     85.8 / 70.2 / 51.7, 1 x 16 over 8192 29.9 / 28.9 / 27.5;
-  //   2 for at most 128 rows a kv head, where 256-row workgroups are half
-  //     empty: 16 x 32 over 4000 100.2 / 81.5 (int4 111.7 / 97.4);
-  //   2 where 128-row workgroups still fit the CUs once: 1 x 1000 51.4 / 42.6,
-  //     1 x 1024 over 3000 124.5 / 113.8; int8 also where they do not but the
-  //     key split below would cut the 256-row ones; 4 x 400 (224 workgroups
-  //     of 256 rows, no split) is 35.5 / 47.6. int4 pays a second barrier a
-  //     round: 1 x 1000 60.2 / 55.2, but 1 x 1024 over 3000 149.3 / 154.9.
-  // Then the key split over workgroups for what is still short of one per CU;
-  // a split keeps at least two rounds of tiles. With two key groups a split
-  // must pay for its partials (every row's written and read again): to the
-  // nearest count, not the next.
-  p.key_groups = 1;
-  int64_t base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
-  const int max_groups = sai::prefill_max_key_groups(D, c->desc.quant);
-  const bool few = c->desc.quant == SAI_KV_INT8
-                       ? base_wgs <= 128 || (base_wgs < 256 && key_tiles >= 16)
-                       : base_wgs <= 128 && key_tiles <= 32;
-  if (max_groups >= 4 && (int64_t)sq * G <= 32)
-    p.key_groups = 4;
-  else if (max_groups >= 2 && ((int64_t)sq * G <= 128 || few))
-    p.key_groups = 2;
-  base_wgs = (int64_t)sai::prefill_workgroups(p, D, G);
-  int nks = 1;
-  if (base_wgs < 256 && key_tiles >= 16)
-    nks = (int)std::min<int64_t>((256 + (p.key_groups == 2 ? base_wgs / 2 : base_wgs - 1)) / base_wgs,
-                                 key_tiles / std::max(4, 2 * p.key_groups));
+  // The work split (prefill_plan). A split of the key range writes partials,
+  // which the decode's combine kernel merges (each row of the chunk a sequence
+  // of its own).
+  sai::PrefillShape shape{};
+  shape.head_dim = sai::stored_head_dim(D);
+  shape.int4 = c->desc.quant == SAI_KV_INT4;
+  shape.group = G;
+  shape.kv_heads = c->desc.num_kv_heads;
+  shape.batch = batch;
+  shape.sq = sq;
+  for (int b = 0; b < batch; ++b) shape.past = std::max<int64_t>(shape.past, c->h_seq_lens[b]);
+  shape.window = p.window;
+  shape.cus = ctx->num_cus;
+  const sai::PrefillPlan plan = sai::prefill_plan(shape);
+  p.key_groups = plan.key_groups;
+  const int nks = plan.key_splits;
   if (nks > 1) {
     p.nksplit = nks;
-    p.ksplit_tiles = (int)((key_tiles + nks - 1) / nks);
+    p.ksplit_tiles = plan.split_tiles;
     const size_t rows = (size_t)batch * sq;
     const size_t need =
         rows * nks * c->desc.num_kv_heads * G * (size_t)(sai::stored_head_dim(D) + 2);

@@ -390,8 +390,6 @@ hipError_t launch_gqa_decode(const DecodeParams& p, int head_dim, int group, int
 hipError_t launch_gqa_prefill(const PrefillParams& p, int head_dim, int group, int quant,
                               hipStream_t s);
 // Workgroups of one prefill launch (the size of PrefillParams::prec_flags).
-// Key groups the prefill kernel has for a cache: up to 1, 2 or 4.
-int prefill_max_key_groups(int head_dim, int quant);
 size_t prefill_workgroups(const PrefillParams& p, int head_dim, int group);
 // Split-partial merge of the decode kernels (gqa_decode.hip).
 hipError_t launch_decode_combine(const DecodeParams& p, int head_dim, int group, hipStream_t st);

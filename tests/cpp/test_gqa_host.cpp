@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../oracle/sai_oracle.h"
+#include "../../smallaios_amd/csrc/prefill_plan.h"
 #include "../../smallaios_amd/host/gqa_host.hpp"
 #include "../../smallaios_amd/host/gqa_session.hpp"
 #include "../../smallaios_amd/host/kv_compression.hpp"
@@ -1511,6 +1512,69 @@ void gpu_cache_sliding_window() {
   REQUIRE(lp.start_token == 2 && lp.token_count == 4, "nothing pending: same view");
 }
 
+// The prefill's work split (prefill_plan.h): every tile that the kernel's row
+// blocks read lies in a split, whatever the sequence's own length; one round
+// of workgroups where the range is split; and the calls that thresholds on the
+// number of workgroups sent to a second round or to key groups that cost more
+// than they gave.
+void cpu_prefill_plan() {
+  using namespace sai;
+  std::mt19937_64 rng(7);
+  auto pick = [&](std::initializer_list<int> l) { return l.begin()[rng() % l.size()]; };
+  for (int it = 0; it < 200000; ++it) {
+    PrefillShape s{};
+    s.int4 = rng() % 2;
+    s.head_dim = s.int4 ? pick({64, 128, 256}) : pick({64, 128, 192, 256});
+    s.group = pick({1, 2, 4, 8});
+    s.kv_heads = pick({1, 2, 3, 8, 16});
+    s.batch = pick({1, 1, 2, 5, 16, 40});
+    s.sq = 1 + (int)(rng() % pick({4, 40, 300, 2100}));
+    s.past = rng() % pick({1, 100, 2000, 20000});
+    s.window = rng() % 2 ? 0 : 1 + (int)(rng() % pick({70, 300, 5000}));
+    s.cus = 256;
+    const PrefillPlan p = prefill_plan(s);
+    const int kg = p.key_groups;
+    REQUIRE(kg == 1 || kg == 2 || (kg == 4 && !s.int4), "groups %d", kg);
+    REQUIRE(kg <= prefill_max_key_groups(s.head_dim, s.int4), "groups %d at %d", kg, s.head_dim);
+    const int qt = prefill_workgroup_rows(s.head_dim, kg) / s.group;
+    const int64_t wgs = (int64_t)((s.sq + qt - 1) / qt) * s.kv_heads * s.batch;
+    REQUIRE(qt >= 1 && p.key_splits >= 1, "%d positions, %d splits", qt, p.key_splits);
+    if (p.key_splits == 1) continue;
+    REQUIRE(wgs * p.key_splits <= s.cus, "%lld x %d workgroups", (long long)wgs, p.key_splits);
+    REQUIRE(p.split_tiles >= std::max(4, 2 * kg), "%d tiles a split", p.split_tiles);
+    // the kernel's tiles of each row block, of lengths up to the longest
+    int64_t most = 0;
+    for (int k = 0; k < 6; ++k) {
+      const int64_t past = k == 0 ? s.past : (int64_t)(rng() % (s.past + 1));
+      for (int q0 = 0; q0 < s.sq; q0 += qt) {
+        const int64_t lo = s.window > 0 ? std::max<int64_t>(0, past + q0 - s.window + 1) / 64 : 0;
+        most = std::max(most, (past + std::min(q0 + qt, s.sq) - 1) / 64 + 1 - lo);
+      }
+    }
+    REQUIRE((int64_t)p.key_splits * p.split_tiles >= most, "%d splits of %d tiles, %lld read",
+            p.key_splits, p.split_tiles, (long long)most);
+    REQUIRE((int64_t)(p.key_splits - 2) * p.split_tiles < most, "empty splits");
+  }
+  // int8, 32Q/8KV
+  struct Call {
+    int batch, sq, past, window, d, key_groups;
+    bool split;
+  };
+  for (const Call& c :
+       {Call{6, 256, 4000, 0, 128, 1, false}, Call{3, 512, 4000, 0, 128, 1, false},
+        Call{5, 250, 4000, 0, 64, 1, false}, Call{1, 1900, 0, 0, 128, 1, false},
+        Call{1, 1000, 4000, 0, 64, 1, true}, Call{1, 1000, 0, 0, 128, 2, false},
+        Call{1, 200, 4000, 0, 64, 1, true}, Call{1, 300, 4000, 0, 128, 2, true},
+        Call{20, 32, 4000, 0, 128, 2, false}, Call{8, 5, 4000, 0, 128, 4, true},
+        Call{8, 5, 8000, 64, 128, 4, false}, Call{1, 1000, 8000, 512, 128, 2, false},
+        Call{2048, 8, 4000, 0, 128, 4, false}, Call{2, 2048, 6144, 0, 128, 1, false}}) {
+    const PrefillPlan p = prefill_plan({c.d, false, 4, 8, c.batch, c.sq, c.past, c.window, 256});
+    REQUIRE(p.key_groups == c.key_groups && (p.key_splits > 1) == c.split,
+            "%d x %d over %d, window %d: %d key groups, %d splits", c.batch, c.sq, c.past,
+            c.window, p.key_groups, p.key_splits);
+  }
+}
+
 int main(int argc, char** argv) {
   struct Case {
     const char* name;
@@ -1523,6 +1587,7 @@ int main(int argc, char** argv) {
       {"cpu_validate", false, cpu_validate},
       {"cpu_errors_and_types", false, cpu_errors_and_types},
       {"cpu_layer_kinds_for_gemma", false, cpu_layer_kinds_for_gemma},
+      {"cpu_prefill_plan", false, cpu_prefill_plan},
       {"gpu_cache_allocate_and_append", true, gpu_cache_allocate_and_append},
       {"gpu_cache_multiple_tokens", true, gpu_cache_multiple_tokens},
       {"gpu_cache_reset", true, gpu_cache_reset},

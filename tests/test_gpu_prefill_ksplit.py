@@ -1,5 +1,5 @@
 """Prefill of short chunks over long pasts, where the host cuts the rows' key
-range into splits (fewer than 256 workgroups, at least 16 tiles to stream):
+range into splits (prefill_plan.h; at least 16 tiles to stream):
 each workgroup streams its split's tiles and writes (m, l, o) partials, and the
 decode's combine kernel merges them, every row of the chunk as a sequence of
 its own. Against the oracle at the prefill bar (2e-3 abs + 1e-2 rel; bf16
@@ -39,6 +39,11 @@ CASES = [
     (S.KV_INT4, 8, 4, 256, [3000, 100], 20, 0, "f32", False),
     (S.KV_INT8, 16, 4, 128, [2500, 0, 1200], 90, 300, "bf16", False),
     (S.KV_INT4, 16, 2, 64, [7000], 8, 0, "f32", True),
+    # chunks of more than 128 rows a kv head that keep one key group
+    (S.KV_INT8, 8, 2, 64, [4000, 3900, 70, 1500], 200, 0, "f32", True),
+    (S.KV_INT8, 8, 2, 128, [4000, 2000, 3999, 100], 400, 0, "bf16", False),
+    (S.KV_INT4, 8, 2, 64, [2000, 1000], 400, 0, "f32", False),
+    (S.KV_INT4, 8, 2, 128, [4000, 10, 500, 3000], 200, 0, "f32", True),
 ]
 
 
@@ -91,3 +96,22 @@ def test_prefill_key_split_repeated_and_reused(rt):
     b = c.gpu_prefill(q, "f32")
     assert np.array_equal(a, b)
     assert_close(a, c.oracle_attend(q), "prefill key split, first")
+
+
+@pytest.mark.parametrize("quant,hq,hkv,d,new,window", [
+    (S.KV_INT8, 8, 2, 128, 8, 1100), (S.KV_INT8, 4, 2, 64, 70, 1087), (S.KV_INT8, 4, 2, 168, 40, 1300),
+    (S.KV_INT8, 8, 1, 256, 9, 1024), (S.KV_INT4, 8, 2, 128, 24, 1500), (S.KV_INT4, 2, 1, 256, 30, 1216)])
+def test_prefill_key_split_window(rt, quant, hq, hkv, d, new, window):
+    """A window much shorter than the past: the splits share the tiles that the
+    window's keys can touch, wherever it lies between two tiles, and sequences
+    that end before the window or the longest one does."""
+    past = [3000, 3007, 3016, 3071, 1601, 20]
+    log(f"prefill key split, window {window}: quant {quant} hq {hq} hkv {hkv} d {d} new {new}")
+    c = Case(rt, 0x4B8 + d + new, len(past), hq, hkv, d, past, new, theta=5e5, quant=quant,
+             permute_pages=True)
+    c.step_kv()
+    q = c.query("f32")
+    got = c.gpu_prefill(q, "f32", window=window)
+    ref = c.oracle_attend(q, mask_window=window)
+    log(f"  worst err/tol {err_tol_ratio(got, ref):.4f}")
+    assert_close(got, ref, "prefill key split, window")

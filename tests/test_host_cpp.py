@@ -3,7 +3,8 @@
 tests/cpp/test_gqa_host (built by __graft_entry__.build()).
 
 The CPU case covers attribute parsing, gqa_validate's messages
-(onnx-rt/src/ops/microsoft.rs:933-984) and the error types. The GPU case runs,
+(onnx-rt/src/ops/microsoft.rs:933-984), the error types and the prefill's work
+split (smallaios_amd/csrc/prefill_plan.h). The GPU case runs,
 in one child process, the restated reference cache tests
 (onnx-rt/tests/test_cuda.rs:1124-1375), the first-token GQA tests
 (test_cuda.rs:3426-3525), dispatch_gqa's error contract, multi-layer
