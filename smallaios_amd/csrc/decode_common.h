@@ -307,6 +307,21 @@ __device__ __forceinline__ void load16(const void* base, size_t off, int dtype, 
   }
 }
 
+// The parameters lie in three 64-byte lines of the kernel-argument memory.
+// Loaded where each is used, those behind the branches of decode_work_item
+// were a memory round trip of their own: 0.1 to 0.2 us of a call. So one of
+// each line, and those that the first loads need, are asked for together at
+// the start (int8, us per call: 1 x 512, 8Q/2KV, 64, 7.66 -> 7.52; 7 x 200..1900,
+// 32Q/8KV, 128, 12.06 -> 11.83; the Gemma 3 4B window layer 14.33 -> 14.12; 16 x
+// 8192 the same). The int4 kernel does without: its short calls gain as much
+// (14 x 72 9.53 -> 9.33), but its long ones lose 1 % at lengths of 2^14 and 2^15
+// (4 x 32768 34.2 -> 34.5).
+__device__ __forceinline__ void load_params(const DecodeParams& p) {
+  __asm__ volatile("" ::"s"(p.kv_heads), "s"(p.uniform_nsplit), "s"(p.window), "s"(p.page_table),
+                   "s"(p.seq_lens), "s"(p.max_pages), "s"(p.pending), "s"(p.split_tokens),
+                   "s"(p.k_new), "s"(p.q), "s"(p.q_dtype), "s"(p.pool));
+}
+
 // (sequence, split) of a decode workgroup and its split's length in 64-token
 // tiles. Uniform split count: direct mapping, splits of split_tokens.
 // Ragged: the host's table of work items (p.ordered), or for larger batches a

@@ -343,6 +343,7 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
   const int work = blockIdx.x;
 
   // ---- (sequence, split) of this workgroup ------------------------------------
+  load_params(p);
   int b, split, nsplit, split_base, tps;
   decode_work_item(p, work, lane, b, split, nsplit, split_base, tps);
   if (b < 0 || b >= p.batch) return;  // uniform over the workgroup
