@@ -456,7 +456,11 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
   // would only take issue slots from the waves that have one). Everything from
   // the first tile's loads on is inside, so that no join lies between them and
   // their uses (at a join the compiler waits for all loads of either path).
-  if (have_first) {
+  // At the stored width 192, which loads its first tile after the query, every
+  // wave prepares the query: behind the branch it took 0.3 us longer (14 x 351,
+  // 8Q/8KV, 15.0 against 14.7 us; 2 x 634..5076 with a window 14.7 against 14.4),
+  // and short sequences gained 0.1. At 256 the two are even.
+  if (D == 192 || have_first) {
   TileRegs<D> TA;
   if constexpr (!BIG)
     load_tile<D>(TA, p.pool, sm_pg, first, p.num_pages, kvh, r, g, n_pages_split);
@@ -620,7 +624,7 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
     // phase: the next tile's K (and scales) load as soon as this tile's QK is
     // issued, its V as soon as this tile's PV is (the last tile reloads
     // itself, so the code stays straight-line)
-    {
+    if (have_first) {
       int cur = first;
       ld(TA, cur);
       for (;;) {
@@ -640,7 +644,7 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
     }
   }
 
-  }  // have_first
+  }  // D == 192 || have_first
 
   // ---- merge the NW waves of the workgroup --------------------------------------
   __shared__ float sm_m[NW][G];
