@@ -147,12 +147,12 @@ __device__ __forceinline__ void reset_ticket(int* counter) {
 }
 
 // Online merge of the splits' (m, l, o) entries for one (head, dim) into
-// (M, Ls, O), C splits per round trip, in split order, skipping split `own`
-// (-1: none) and splits with no visible key; `ph` points at split 0's (m, l,
-// o[...]) block of this head, `stride` floats apart per split, `d` the dim.
+// (M, Ls, O), C splits per round trip, in split order, skipping splits with no
+// visible key; `ph` points at split 0's (m, l, o[...]) block of this head,
+// `stride` floats apart per split, `d` the dim.
 template <int C>
 __device__ __forceinline__ void merge_partials(const float* ph, size_t stride, int d, int nsplit,
-                                               int own, float& M, float& Ls, float& O) {
+                                               float& M, float& Ls, float& O) {
   for (int s0 = 0; s0 < nsplit; s0 += C) {
     float m[C], l[C], o[C];
 #pragma unroll
@@ -166,7 +166,7 @@ __device__ __forceinline__ void merge_partials(const float* ph, size_t stride, i
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int s = s0 + i;
-      if (s >= nsplit || s == own || m[i] == -INFINITY) continue;
+      if (s >= nsplit || m[i] == -INFINITY) continue;
       const float mn = fmaxf(M, m[i]);
       const float fa = M == -INFINITY ? 0.0f : fast_exp2(M - mn);
       const float fb = fast_exp2(m[i] - mn);
@@ -258,24 +258,33 @@ __device__ __forceinline__ void merge_splits_by(const float* p0, size_t stride, 
 template <int D, int G, int NT, class F>
 __device__ __forceinline__ void merge_splits(const float* p0, size_t stride, int nsplit,
                                              float2* sm, F&& store) {
-  if constexpr (G * D <= 64) {
-    // one wave holds every entry: a dim per lane, each reading its own (m, l),
-    // has no barrier in the way (int4, 1 x 4585, 8Q/8KV, D = 64, 9 splits:
-    // 11.96 against 12.60 us per step)
-    const int t = threadIdx.x;
-    if (t < G * D) {
-      float M = -INFINITY, L = 0.0f, O = 0.0f;
-      if (nsplit <= 4)
-        merge_partials<4>(p0, stride, t, nsplit, -1, M, L, O);
-      else if (nsplit <= 8)
-        merge_partials<8>(p0, stride, t, nsplit, -1, M, L, O);
-      else
-        merge_partials<16>(p0, stride, t, nsplit, -1, M, L, O);
-      const float v = L > 0.0f ? O / L : 0.0f;
-      const float next = __int_as_float(swap_pair(__float_as_int(v)));
-      if ((t & 1) == 0) store(0, t, v, next);
+  if constexpr (G * D <= NT) {
+    // An entry per thread, each reading its own (m, l), has no barrier in the
+    // way. One wave (G * D <= 64) always takes it (int4, 1 x 4585, 8Q/8KV, D =
+    // 64, 9 splits: 11.96 against 12.60 us per step), more waves up to 4 splits
+    // (2: int4 2 x 409, 8Q/2KV, 128, 10.7 against 11.05 us, int8 16 x 516, 10.8
+    // against 11.05; 3: int4 3 x 590 11.2 against 11.25; 5: int4 6 x 1200 12.35
+    // against 12.25).
+    if (G * D <= 64 || nsplit <= 4) {
+      const int t = threadIdx.x;
+      if (t < G * D) {
+        const int hd = t / D, d = t % D;
+        const float* ph = p0 + hd * (D + 2);
+        float M = -INFINITY, L = 0.0f, O = 0.0f;
+        if (nsplit <= 2)
+          merge_partials<2>(ph, stride, d, nsplit, M, L, O);
+        else if (nsplit <= 4)
+          merge_partials<4>(ph, stride, d, nsplit, M, L, O);
+        else if (nsplit <= 8)
+          merge_partials<8>(ph, stride, d, nsplit, M, L, O);
+        else
+          merge_partials<16>(ph, stride, d, nsplit, M, L, O);
+        const float v = L > 0.0f ? O / L : 0.0f;
+        const float next = __int_as_float(swap_pair(__float_as_int(v)));
+        if ((d & 1) == 0) store(hd, d, v, next);
+      }
+      return;
     }
-    return;
   }
   if (nsplit <= 4)
     merge_splits_by<D, G, NT, 4>(p0, stride, nsplit, sm, store);

@@ -1428,11 +1428,11 @@ __global__ __launch_bounds__(64 * NW, NW >= 8 ? 2 : 1) void tq_attend_kernel(
       float M = -INFINITY, Ls = 0.0f, O = 0.0f;
       const float* ph = part0 + g * (D + 2);
       if (nsplit <= 4)
-        merge_partials<4>(ph, pstride, i, nsplit, -1, M, Ls, O);
+        merge_partials<4>(ph, pstride, i, nsplit, M, Ls, O);
       else if (nsplit <= 8)
-        merge_partials<8>(ph, pstride, i, nsplit, -1, M, Ls, O);
+        merge_partials<8>(ph, pstride, i, nsplit, M, Ls, O);
       else
-        merge_partials<16>(ph, pstride, i, nsplit, -1, M, Ls, O);
+        merge_partials<16>(ph, pstride, i, nsplit, M, Ls, O);
       sy[g][i] = MODE == 2 ? O : (Ls > 0.0f ? O / Ls : 0.0f);
     }
     if (threadIdx.x == 0) reset_ticket(counter);

@@ -62,6 +62,35 @@ def test_decode_ragged_merges(rt, case):
     assert np.abs(a - b).max() <= 64 * 2.0 ** -24 * 6
 
 
+@pytest.mark.parametrize("quant,hq,hkv,d", [
+    (S.KV_INT8, 1, 1, 64), (S.KV_INT8, 4, 1, 64), (S.KV_INT8, 4, 2, 128), (S.KV_INT8, 4, 1, 128),
+    (S.KV_INT8, 2, 2, 168), (S.KV_INT8, 1, 1, 256), (S.KV_INT4, 2, 2, 64), (S.KV_INT4, 8, 1, 64),
+    (S.KV_INT4, 4, 1, 128), (S.KV_INT4, 8, 1, 128), (S.KV_INT4, 1, 1, 256), (S.KV_INT4, 2, 1, 256)])
+def test_decode_merge_split_counts(rt, quant, hq, hkv, d):
+    """The in-kernel merge over 2 to 17 splits, where its loads' width and its
+    path change (an entry or a pair of dims per thread; heads x head_dim below,
+    at and above a workgroup's threads): against the oracle, and within a few
+    f32 roundings of the combine kernel's merge of the same partials."""
+    prev_split, prev_merge = rt.set_decode_split(64), rt.set_decode_merge(1)
+    try:
+        for n in (2, 3, 4, 5, 8, 9, 16, 17):
+            log(f"decode merge: quant {quant} hq {hq} hkv {hkv} d {d} splits {n}")
+            past = [64 * n - 1, 64 * n - 64]  # the second's last split holds one token
+            c = Case(rt, 0x5D3 + d + n, 2, hq, hkv, d, past, 1, theta=5e5, quant=quant,
+                     permute_pages=True)
+            c.step_kv()
+            q = c.query("f32")
+            rt.set_decode_merge(1)
+            got = c.gpu_decode(q)
+            assert rt.last_decode_shape() == (2 * n * hkv, 64) and rt.last_decode_launches() == 1
+            assert_close(got, c.oracle_attend(q), f"{n} splits")
+            rt.set_decode_merge(0)
+            assert np.abs(got - c.gpu_decode(q)).max() <= 64 * 2.0 ** -24 * 6
+    finally:
+        rt.set_decode_split(prev_split)
+        rt.set_decode_merge(prev_merge)
+
+
 @pytest.mark.parametrize("quant,batch", [(S.KV_INT8, 256), (S.KV_INT8, 257), (S.KV_INT4, 300)])
 def test_decode_many_ragged_sequences(rt, quant, batch):
     """256 sequences take the table of work items, more take the scan."""
