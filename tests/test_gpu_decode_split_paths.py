@@ -91,12 +91,18 @@ def test_decode_merge_split_counts(rt, quant, hq, hkv, d):
         rt.set_decode_merge(prev_merge)
 
 
-@pytest.mark.parametrize("quant,batch", [(S.KV_INT8, 256), (S.KV_INT8, 257), (S.KV_INT4, 300)])
+@pytest.mark.parametrize("quant,batch", [(S.KV_INT8, 65), (S.KV_INT4, 130), (S.KV_INT8, 256),
+                                         (S.KV_INT4, 256), (S.KV_INT8, 257), (S.KV_INT4, 300)])
 def test_decode_many_ragged_sequences(rt, quant, batch):
-    """256 sequences take the table of work items, more take the scan."""
+    """Up to 256 sequences take the table of work items, read 64 entries at a
+    time, more take the scan; both over 1 to several splits a sequence."""
     log(f"decode, {batch} ragged sequences, quant {quant}")
-    lens = [int(x) for x in np.random.default_rng(batch).integers(0, 700, size=batch)]
+    lens = [int(x) for x in np.random.default_rng(batch).integers(0, 1500, size=batch)]
     c = Case(rt, 0x5D2 + batch, batch, 2, 1, 64, lens, 1, theta=1e4, quant=quant)
     c.step_kv()
     q = c.query("f32")
-    assert_close(c.gpu_decode(q), c.oracle_attend(q), "many ragged sequences")
+    got = c.gpu_decode(q)
+    wg, split = rt.last_decode_shape()
+    splits = [(n + split) // split for n in lens]
+    assert wg == sum(splits) and len(set(splits)) > 1  # several splits, not all alike
+    assert_close(got, c.oracle_attend(q), "many ragged sequences")

@@ -54,16 +54,16 @@ def replay_matches(step, out, reps=4):
 
 
 @pytest.mark.parametrize("quant", [S.KV_INT8, S.KV_INT4])
-@pytest.mark.parametrize("split", [0, 256])
-def test_fused_decode_step_graph(rt, quant, split):
-    """sai_gqa_with_cache (append + decode + in-kernel merge) in a graph; the
-    replays rewrite the same pending slot."""
+@pytest.mark.parametrize("split,merge", [(0, 2), (256, 2), (256, 0)])
+def test_fused_decode_step_graph(rt, quant, split, merge):
+    """sai_gqa_with_cache (append + decode, splits merged in-kernel or by the
+    combine kernel) in a graph; the replays rewrite the same pending slot."""
     import torch
-    log(f"graph: fused decode quant={quant} split={split}")
+    log(f"graph: fused decode quant={quant} split={split} merge={merge}")
     lens = [700, 1500, 33]
     c = Case(rt, 0x6A0 + quant + split, len(lens), 16, 4, 128, lens, 0, quant=quant,
              permute_pages=True, extra_tokens=1)
-    prev = rt.set_decode_split(split)
+    prev, prev_m = rt.set_decode_split(split), rt.set_decode_merge(merge)
     try:
         q = c.rng.standard_normal((c.batch, 1, c.hq * c.d), dtype=np.float32)
         k, v = c.kv(1)
@@ -75,11 +75,13 @@ def test_fused_decode_step_graph(rt, quant, split):
                                       c.cos.shape[0], c.do_rotary, c.interleaved, stream=s)
 
         got = replay_matches(step, out)
+        assert rt.last_decode_launches() == (1 if merge else 2)
         c.ocache.append(k, v, c.cos, c.sin, c.do_rotary, c.interleaved)
         ref = c.oracle_attend(to_bf16_f32(q))
         assert np.allclose(got.cpu().numpy(), ref, atol=2e-3, rtol=1e-2)
     finally:
         rt.set_decode_split(prev)
+        rt.set_decode_merge(prev_m)
 
 
 def test_prefill_graph(rt):

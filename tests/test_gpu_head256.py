@@ -48,18 +48,19 @@ def test_decode_d256_groups(rt, quant, hq, hkv):
     c.check_codes(seqs=[1])
 
 
-@pytest.mark.parametrize("split", [64, 1024])
-def test_decode_d256_split_merge_and_fused(rt, quant, split):
-    """Several split partials through the combine kernel, then the fused
-    append + decode step."""
-    log(f"decode d=256 split={split}")
+@pytest.mark.parametrize("split,merge", [(64, 0), (64, 1), (1024, 0), (1024, 2)])
+def test_decode_d256_split_merge_and_fused(rt, quant, split, merge):
+    """Several split partials through the combine kernel and in-kernel, then the
+    fused append + decode step."""
+    log(f"decode d=256 split={split} merge={merge}")
     c = Case(rt, 333, 3, 8, 4, D, [2500, 1, 640], 1, theta=1e6, permute_pages=True,
              extra_tokens=1, quant=quant)
-    prev = rt.set_decode_split(split)
+    prev, prev_m = rt.set_decode_split(split), rt.set_decode_merge(merge)
     try:
         c.step_kv()
         q = c.query()
         assert_close(c.gpu_decode(q), c.oracle_attend(q), f"d=256 split {split}")
+        assert rt.last_decode_launches() == (1 if merge else 2)
         c.cache.advance()
         q = c.query()
         got = c.step_fused(q)
@@ -67,6 +68,7 @@ def test_decode_d256_split_merge_and_fused(rt, quant, split):
         c.check_codes(seqs=[1])
     finally:
         rt.set_decode_split(prev)
+        rt.set_decode_merge(prev_m)
 
 
 def test_decode_d256_windows(rt, quant):

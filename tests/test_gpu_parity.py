@@ -381,7 +381,7 @@ def test_decode_bf16_output(rt, quant):
     contexts (4 sequences), the fused step and the no-alloc step with bf16
     Q and bf16 output, against the f32 oracle within the tolerance widened
     by bf16 rounding; the decoded step's codes stay bit-exact. Split merges
-    in-kernel (uniform) and through the combine kernel (ragged)."""
+    in-kernel (uniform, and ragged as chosen) and through the combine kernel."""
     log(f"decode bf16 output: quant {quant}")
     from _gpu_util import bf16_tol_close
     c = Case(rt, 0x5A1A0B16, 4, 32, 8, 128, [8191] * 4, 1, theta=5e5, quant=quant,
@@ -393,13 +393,23 @@ def test_decode_bf16_output(rt, quant):
     log(f"  uniform 8k: worst err/tol {r:.4f}")
     c.check_codes(seqs=[2])
     c.cache.advance()
-    # ragged lengths: the combine kernel's store
+    # ragged lengths: the merge in the decode kernel, then (over the same token)
+    # the combine kernel's store
     c.cache.set_seq_lens(np.array([8192, 3000, 777, 5000], np.int32))
     c.ocache.seq_len = np.array([8192, 3000, 777, 5000], np.int32)
     q = c.query("bf16")
     got = c.step_fused(q, "bf16", out_dtype="bf16")
-    r = bf16_tol_close(got, c.oracle_attend(q), "bf16 fused step, ragged")
-    log(f"  ragged: worst err/tol {r:.4f}")
+    assert rt.last_decode_launches() == 1
+    ref = c.oracle_attend(q)
+    r = bf16_tol_close(got, ref, "bf16 fused step, ragged")
+    prev = rt.set_decode_merge(0)
+    try:
+        got = c.gpu_decode(q, "bf16", out_dtype="bf16")
+    finally:
+        rt.set_decode_merge(prev)
+    assert rt.last_decode_launches() == 2
+    rc = bf16_tol_close(got, ref, "bf16 step, ragged, combine kernel")
+    log(f"  ragged: worst err/tol {r:.4f}, combine {rc:.4f}")
 
 
 def test_prefill_bf16_output(rt):

@@ -27,13 +27,23 @@ def rt():
     r.close()
 
 
-def test_two_caches_two_streams(rt):
+@pytest.mark.parametrize("merge,launches", [(2, 1), (0, 2)])
+def test_two_caches_two_streams(rt, merge, launches):
     """Interleaved fused decode steps (append + attend + advance) on two
-    int8 caches of different shapes, each on its own stream, both checked
-    against the oracle step by step; the ragged one merges in the combine
-    kernel, the uniform one in-kernel (automatic merge)."""
+    int8 caches of different shapes (one ragged, one uniform), each on its own
+    stream, both checked against the oracle step by step; splits merged
+    in-kernel (as chosen) and by the combine kernel, which reads the split
+    ranges of its own cache."""
+    log(f"two caches, two streams: 3 fused steps each, interleaved, merge {merge}")
+    prev = rt.set_decode_merge(merge)
+    try:
+        two_caches_two_streams(rt, launches)
+    finally:
+        rt.set_decode_merge(prev)
+
+
+def two_caches_two_streams(rt, launches):
     import torch
-    log("two caches, two streams: 3 fused steps each, interleaved")
     a = Case(rt, 0x5711, 4, 32, 8, 128, [3000, 700, 129, 2048], 1, theta=5e5,
              kv_dtype="bf16", permute_pages=True, extra_tokens=3)
     b = Case(rt, 0x5712, 8, 16, 2, 128, [4095] * 8, 1, theta=5e5, kv_dtype="bf16",
@@ -53,6 +63,7 @@ def test_two_caches_two_streams(rt):
             with torch.cuda.stream(s):
                 c.cache.decode_with_cache(0, qd, kd, vd, out, c.batch, c.hq, c.cos_d, c.sin_d,
                                           c.cos.shape[0], stream=s)
+                assert rt.last_decode_launches() == launches
                 c.cache.advance(stream=s)
             outs[name].append((out, qd, kd, vd))
     torch.cuda.synchronize()

@@ -36,14 +36,24 @@ def fused(c, q, k, v, noalloc):
     return out.cpu().numpy()
 
 
+@pytest.mark.parametrize("merge", [2, 0])
 @pytest.mark.parametrize("call", [0, 1])
-def test_noalloc_matches_with_cache(rt, call):
-    # call 0: a uniform 8 x 4096 batch (two splits each, merged in-kernel);
-    # call 1, smaller: a ragged 3-sequence batch at head_dim 64 (combine kernel)
+def test_noalloc_matches_with_cache(rt, call, merge):
+    """call 0: a uniform 8 x 4096 batch (two splits each); call 1, smaller: a
+    ragged 3-sequence batch at head_dim 64. Both merge in-kernel as chosen, and
+    through the combine kernel (the split ranges in the fixed scratch)."""
+    prev = rt.set_decode_merge(merge)
+    try:
+        noalloc_matches_with_cache(rt, call, 1 if merge else 2)
+    finally:
+        rt.set_decode_merge(prev)
+
+
+def noalloc_matches_with_cache(rt, call, launches):
     shapes = [dict(batch=8, hq=32, hkv=8, d=128, past=[4095] * 8),
               dict(batch=3, hq=16, hkv=4, d=64, past=[500, 77, 1200])]
     sh = shapes[call]
-    log(f"noalloc call {call}: {sh}")
+    log(f"noalloc call {call}, {launches} launches: {sh}")
     seed = 0xA110C + call
     cases = [Case(rt, seed, sh["batch"], sh["hq"], sh["hkv"], sh["d"], sh["past"], 1, theta=5e5,
                   kv_dtype="bf16", permute_pages=True, extra_tokens=1) for _ in range(2)]
@@ -51,7 +61,9 @@ def test_noalloc_matches_with_cache(rt, call):
     kv = [c.kv(1) for c in cases]
     assert np.array_equal(q[0], q[1]) and np.array_equal(kv[0][0], kv[1][0])
     want = fused(cases[0], q[0], *kv[0], noalloc=False)
+    assert rt.last_decode_launches() == launches
     got = fused(cases[1], q[1], *kv[1], noalloc=True)
+    assert rt.last_decode_launches() == launches
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), \
         f"noalloc differs from with_cache, call {call}: max |diff| {np.abs(got - want).max():.3e}"
     assert_close(got, want, f"noalloc vs with_cache, call {call}")
