@@ -26,6 +26,7 @@
 // workgroup, otherwise by the workgroup that stores the last split partial.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "decode_common.h"
@@ -252,16 +253,19 @@ __device__ __forceinline__ float wave_qjl(const uint32_t (&code)[D / 64], float 
 
 // Encodes the row x (lane l: dims l + 64 e) as position r of (kv head h,
 // sequence b), K (kind 0) or V (kind 1), and stores it: K codes row-major; V
-// codes into the position's bits of its tile, by read-modify-write of the
-// words in memory (the caller guarantees that no other wave writes that tile
-// meanwhile);
+// codes into the position's bits of its tile, in the LDS copy `stile` of the
+// tile's words when given, else by read-modify-write of the words in memory
+// (the caller guarantees that no other wave writes that tile meanwhile);
 // then the parameters (scale, zero point, QJL mean, sum of the codes) and the
-// QJL sign words. Orders its LDS use at wave level only.
+// QJL sign words. Orders its LDS use at wave level only. (Without `stile` the
+// attention instances that call this get other registers: head_dim 256, 3
+// bits, group 2 spilled 12 SGPRs instead of 8 and took 57.7 instead of 54.3 us
+// at 16 x 8191.)
 template <int D, int BITS>
 __device__ __forceinline__ void wave_store_row(const TqArgs& a, const float (&x)[D / 64],
                                                const float (&sgn)[D / 64], int lane, int h, int b,
-                                               int r, int kind, float* sres,
-                                               uint32_t* scode) {
+                                               int r, int kind, uint32_t (*stile)[2 * BITS + 1],
+                                               float* sres, uint32_t* scode) {
 #pragma clang fp contract(off)
   constexpr int E = D / 64;
   constexpr int W = D * BITS / 32;  // K code words per row
@@ -296,7 +300,7 @@ __device__ __forceinline__ void wave_store_row(const TqArgs& a, const float (&x)
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int d = lane + 64 * e;
-      uint32_t* tw = vt + d * TBW;
+      uint32_t* tw = stile ? stile[d] : vt + d * TBW;
       tw[w] = (tw[w] & ~(LEVELS << sh)) | (code[e] << sh);
       if (sh + BITS > 32) tw[w + 1] = (tw[w + 1] & ~(LEVELS >> (32 - sh))) | (code[e] >> (32 - sh));
     }
@@ -314,6 +318,47 @@ __device__ __forceinline__ void wave_store_row(const TqArgs& a, const float (&x)
     }
   }
   if (lane == 0) (kind ? a.par_v : a.par_k)[row] = make_float4(scale, zero, c, csum);
+}
+
+// ---- write of one position: one wave per (sequence, kv head, K|V) ------------
+// A row's arithmetic over the 64 lanes, the tile's V words through LDS. The
+// tile kernel below has a row in D/32 lanes, which pays from two rows on; one
+// alone took it 7.9 us a call and takes 4.9 here (1 sequence, 8 kv heads, D =
+// 256, 4 bits, QJL; 128: 6.8 and 4.7).
+template <int D, int BITS>
+__global__ __launch_bounds__(64) void tq_write_row_kernel(const TqArgs a, const void* k,
+                                                          const void* v, int bf16) {
+  constexpr int E = D / 64;
+  const int lane = threadIdx.x;
+  const int kind = blockIdx.x & 1, h = blockIdx.x >> 1, b = blockIdx.y;
+  __shared__ uint32_t scode[D];
+  __shared__ float sres[D];
+  const void* src = kind ? v : k;
+  const size_t in_off = ((size_t)b * a.heads + h) * D;
+  float x[E], sgn[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    x[e] = load_row_elem(src, in_off + lane + 64 * e, bf16 != 0);
+    sgn[e] = (float)a.signs[(size_t)h * D + lane + 64 * e];
+  }
+  __shared__ uint32_t stile[D][2 * BITS + 1];
+  const int r = a.seq_lens[b];
+  uint32_t* vt = (uint32_t*)(a.codes_v + (((size_t)h * a.batch_cap + b) * a.tiles_cap + r / 64) *
+                                             tq_vtile_bytes(D, BITS));
+  const int w_lo = (r % 64 * BITS) >> 5, w_hi = (r % 64 * BITS + BITS - 1) >> 5;
+  if (kind) {
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      for (int w = w_lo; w <= w_hi; ++w) stile[lane + 64 * e][w] = vt[(lane + 64 * e) * 2 * BITS + w];
+    wave_lds_sync();
+  }
+  wave_store_row<D, BITS>(a, x, sgn, lane, h, b, r, kind, stile, sres, scode);
+  if (kind) {
+    wave_lds_sync();
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      for (int w = w_lo; w <= w_hi; ++w) vt[(lane + 64 * e) * 2 * BITS + w] = stile[lane + 64 * e][w];
+  }
 }
 
 // ---- write: one workgroup per (sequence, kv head, K|V, 64-position tile) ----
@@ -380,15 +425,15 @@ __global__ __launch_bounds__(2 * D) void tq_write_kernel(const TqArgs a, const v
   constexpr uint32_t LEVELS = (1u << BITS) - 1u;
   constexpr int STRIDE = D / 4 + 1;  // dwords of a row of codes in LDS
   const int tid = threadIdx.x, lane = tid & 63;
-  const int j = tid % L, pr = tid / L;  // dims 32j .. 32j+31 of tile position pr
   const int kind = blockIdx.y & 1, h = blockIdx.y >> 1, b = blockIdx.z;
   const int len = a.seq_lens[b];
   const int tile = len / 64 + (int)blockIdx.x;
   const int r_lo = max(len, tile * 64), r_hi = min(len + s_new, tile * 64 + 64);
   if (r_lo >= r_hi) return;  // uniform
   __shared__ uint32_t scode[64 * STRIDE];  // V: a byte per code, [position][dim]
-  const int r = tile * 64 + pr;
-  const bool live = r >= r_lo && r < r_hi;
+  const int j = tid % L, r = r_lo + tid / L;  // dims 32j .. 32j+31 of position r
+  const int pr = r - tile * 64;               // (past the tile: not live)
+  const bool live = r < r_hi;
   if (__ballot(live) != 0) {
     const void* src = kind ? v : k;
     // a lane outside the pass encodes its first row (and stores nothing)
@@ -489,7 +534,8 @@ __global__ __launch_bounds__(2 * D) void tq_write_kernel(const TqArgs a, const v
     const size_t row = ((size_t)h * a.batch_cap + b) * a.rows_cap + r;
     if (kind) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) scode[pr * STRIDE + 8 * j + i] = cb[i];
+      for (int i = 0; i < 8; ++i)
+        if (live) scode[pr * STRIDE + 8 * j + i] = cb[i];
     } else {
       uint32_t wd[BITS] = {};
 #pragma unroll
@@ -539,13 +585,14 @@ __global__ __launch_bounds__(2 * D) void tq_write_kernel(const TqArgs a, const v
   }
   if (!kind) return;  // uniform
   __syncthreads();
-  // four dims' word w of the tile per thread
+  // four dims' word w of the tile per thread, of those that the pass touches
   uint32_t* vt = (uint32_t*)(a.codes_v + (((size_t)h * a.batch_cap + b) * a.tiles_cap + tile) *
                                              tq_vtile_bytes(D, BITS));
   const int lo = r_lo - tile * 64, hi = r_hi - tile * 64;
+  const int w_lo = (lo * BITS) >> 5, nw = ((hi * BITS - 1) >> 5) - w_lo + 1;
   constexpr int NP = (31 + BITS - 1) / BITS + 1;  // positions with bits in a word, at most
-  for (int it = tid; it < D / 4 * TBW; it += 2 * D) {
-    const int w = it % TBW, d4 = it / TBW;
+  for (int it = tid; it < D / 4 * nw; it += blockDim.x) {
+    const int w = w_lo + it % nw, d4 = it / nw;
     const int i0 = (32 * w) / BITS;
     uint32_t mask = 0u, wd[4] = {};
 #pragma unroll
@@ -1160,8 +1207,8 @@ __global__ __launch_bounds__(64 * NW, NW >= 8 ? 2 : 1) void tq_attend_kernel(
       float sgn[D / 64];
 #pragma unroll
       for (int e = 0; e < D / 64; ++e) sgn[e] = (float)a.signs[(size_t)kvh * D + lane + 64 * e];
-      wave_store_row<D, BITS>(a, xnk, sgn, lane, kvh, b, L - 1, 0, sres[wave], scode);
-      wave_store_row<D, BITS>(a, xnv, sgn, lane, kvh, b, L - 1, 1, sres[wave], scode);
+      wave_store_row<D, BITS>(a, xnk, sgn, lane, kvh, b, L - 1, 0, nullptr, sres[wave], scode);
+      wave_store_row<D, BITS>(a, xnv, sgn, lane, kvh, b, L - 1, 1, nullptr, sres[wave], scode);
       __threadfence_block();
       tq_load_tile<D, BITS, MODE>(a, rbase, vbase, first, r1, lane, tb[0]);
     }
@@ -1490,6 +1537,13 @@ hipError_t dispatch_dbits(int d, int bits, F&& f) {
 hipError_t launch_tq_write(const TqArgs& a, const void* k, const void* v, int bf16, int batch,
                            int s_new, hipStream_t st) {
   if (batch <= 0 || s_new <= 0) return hipSuccess;
+  if (s_new == 1)
+    return dispatch_dbits(a.head_dim, a.bits, [&](auto dd, auto bb) -> hipError_t {
+      constexpr int D = decltype(dd)::value, B = decltype(bb)::value;
+      hipLaunchKernelGGL((tq_write_row_kernel<D, B>), dim3(2 * a.heads, batch), dim3(64), 0, st, a,
+                         k, v, bf16);
+      return hipGetLastError();
+    });
   // 16-byte loads of a lane's 32 dims need both inputs aligned (a row is a
   // multiple of 64 bytes); the elementwise loads serve the others
   const int vec = (((uintptr_t)k | (uintptr_t)v) & 15u) == 0;
@@ -1497,7 +1551,14 @@ hipError_t launch_tq_write(const TqArgs& a, const void* k, const void* v, int bf
   const dim3 grid((s_new + 126) / 64, 2 * a.heads, batch);
   return dispatch_dbits(a.head_dim, a.bits, [&](auto dd, auto bb) -> hipError_t {
     constexpr int D = decltype(dd)::value, B = decltype(bb)::value;
-    hipLaunchKernelGGL((tq_write_kernel<D, B>), grid, dim3(2 * D), 0, st, a, k, v, bf16, vec,
+    // The waves that a tile's rows of this pass need, and two from 8 rows on for
+    // the V words. A workgroup for all 64 positions left one a CU, mostly idle:
+    // 16 x 2 rows (8 kv heads, D = 256, 8 bits) 16.0 us against 9.0, 64 x 5 (128,
+    // 4 bits) 19.9 against 10.1, 16 x 8 (256, 4 bits) 15.9 against 9.1; 1 x 16
+    // (128) 8.4 us in one wave, 7.2 in two.
+    const int rows = std::min(s_new, 64) * (D / 32);
+    const int threads = std::max(s_new >= 8 ? 128 : 64, (rows + 63) / 64 * 64);
+    hipLaunchKernelGGL((tq_write_kernel<D, B>), grid, dim3(threads), 0, st, a, k, v, bf16, vec,
                        s_new);
     return hipGetLastError();
   });

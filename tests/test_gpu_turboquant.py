@@ -157,8 +157,9 @@ def test_writes_across_tile_boundaries(rt, d, bits):
                                                (128, 4, True, 3), (128, 8, False, 2),
                                                (256, 3, False, 0), (256, 4, True, 1)])
 def test_write_rows_at_tile_edges(rt, d, bits, bf16, shift):
-    """Passes of 1, 62, 1, 64, 65, 16 and 17 rows: starts and ends at, before
-    and after the 64-position tiles and the rows of a wave. The inputs start
+    """Passes of 1, 62, 1, 64, 65, 16, 17, 2, 3 and 30 rows: starts and ends at,
+    before and after the 64-position tiles and the rows of a wave; one row takes
+    a kernel of its own. The inputs start
     `shift` elements into their buffer, so the elementwise loads of inputs
     that are not 16-byte aligned run too, and hold rows of zeros of both
     signs, of one value, and one-hot rows. Every row bit for bit."""
@@ -166,7 +167,7 @@ def test_write_rows_at_tile_edges(rt, d, bits, bf16, shift):
     log(f"tq write edges d={d} bits={bits} bf16={bf16} shift={shift}")
     rng = np.random.default_rng(d + 7 * bits + shift)
     batch, heads = 2, 3
-    sizes = (1, 62, 1, 64, 65, 16, 17)
+    sizes = (1, 62, 1, 64, 65, 16, 17, 2, 3, 30)
     c = S.TqCache(rt, 1, heads, d, bits, True, batch, sum(sizes), seed=SEED)
     try:
         ks, vs = [], []
