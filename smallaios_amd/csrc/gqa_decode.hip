@@ -461,143 +461,142 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
   // 8Q/8KV, 15.0 against 14.7 us; 2 x 634..5076 with a window 14.7 against 14.4),
   // and short sequences gained 0.1. At 256 the two are even.
   if (D == 192 || have_first) {
-  TileRegs<D> TA;
-  if constexpr (!BIG)
-    load_tile<D>(TA, p.pool, sm_pg, first, p.num_pages, kvh, r, g, n_pages_split);
-  // Tile first + slots (the one this wave most likely takes next, never the
-  // appender's; else the first tile again) is touched (one dword per 128-byte
-  // line) so that it streams into L2 while the query is prepared, instead of
-  // the memory pipe idling until the loop issues its load. The values are
-  // consumed only where the first tile is needed anyway. Branch-free (lanes
-  // past the last line repeat it).
-  constexpr int kLines = (int)(block_bytes_int8(D) / 128);  // 33 for D = 128
-  constexpr int kTouch = (4 * kLines + 63) / 64;              // loads per lane
-  uint32_t touch[kTouch];
+    TileRegs<D> TA;
+    if constexpr (!BIG)
+      load_tile<D>(TA, p.pool, sm_pg, first, p.num_pages, kvh, r, g, n_pages_split);
+    // Tile first + slots (the one this wave most likely takes next, never the
+    // appender's; else the first tile again) is touched (one dword per 128-byte
+    // line) so that it streams into L2 while the query is prepared, instead of
+    // the memory pipe idling until the loop issues its load. The values are
+    // consumed only where the first tile is needed anyway. Branch-free (lanes
+    // past the last line repeat it).
+    constexpr int kLines = (int)(block_bytes_int8(D) / 128);  // 33 for D = 128
+    constexpr int kTouch = (4 * kLines + 63) / 64;              // loads per lane
+    uint32_t touch[kTouch];
 #pragma unroll
-  for (int j = 0; j < kTouch; ++j) touch[j] = 0;
-  if constexpr (!BIG) {
-    const int t1 = first + slots < pool_end ? first + slots : first;
+    for (int j = 0; j < kTouch; ++j) touch[j] = 0;
+    if constexpr (!BIG) {
+      const int t1 = first + slots < pool_end ? first + slots : first;
 #pragma unroll
-    for (int j = 0; j < kTouch; ++j) {
-      const int line = min(lane + 64 * j, 4 * kLines - 1);
-      const int pg = sm_pg[min(t1 * 4 + line / kLines, n_pages_split - 1)];
-      const uint8_t* a = p.pool + block_offset(pg, kvh, p.num_pages, block_bytes_int8(D)) +
-                         (size_t)(line % kLines) * 128;
-      touch[j] = *(const uint32_t*)a;
+      for (int j = 0; j < kTouch; ++j) {
+        const int line = min(lane + 64 * j, 4 * kLines - 1);
+        const int pg = sm_pg[min(t1 * 4 + line / kLines, n_pages_split - 1)];
+        const uint8_t* a = p.pool + block_offset(pg, kvh, p.num_pages, block_bytes_int8(D)) +
+                           (size_t)(line % kLines) * 128;
+        touch[j] = *(const uint32_t*)a;
+      }
     }
-  }
 
-  // ---- Q: RoPE at position L-1, split into three int8 terms ------------------
-  // y = sq * (hi + mid / 254 + lo / 254^2), sq = max|y| / 127 over the head:
-  // ~24 significant bits, about f32's own. (Two terms, ~16 bits, put keys
-  // with x20 outlier channels at 0.96 of the output tolerance: their score
-  // terms reach the hundreds.) Each lane packs its own term t; t = 3 is zero.
-  v4i qB[NP][KS];
-  float qw[NP];
+    // ---- Q: RoPE at position L-1, split into three int8 terms ------------------
+    // y = sq * (hi + mid / 254 + lo / 254^2), sq = max|y| / 127 over the head:
+    // ~24 significant bits, about f32's own. (Two terms, ~16 bits, put keys
+    // with x20 outlier channels at 0.96 of the output tolerance: their score
+    // terms reach the hundreds.) Each lane packs its own term t; t = 3 is zero.
+    v4i qB[NP][KS];
+    float qw[NP];
 #pragma unroll
-  for (int ps = 0; ps < NP; ++ps) {
-    const bool live = 4 * ps + (r >> 2) < G;
-    float qv[KS][16];
-    float amax = 0.0f;
+    for (int ps = 0; ps < NP; ++ps) {
+      const bool live = 4 * ps + (r >> 2) < G;
+      float qv[KS][16];
+      float amax = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int c0 = kdim0<D>(g, ks);  // first dim of this lane's chunk
-      float x[16];
+      for (int ks = 0; ks < KS; ++ks) {
+        const int c0 = kdim0<D>(g, ks);  // first dim of this lane's chunk
+        float x[16];
 #pragma unroll
-      for (int i = 0; i < 16; ++i) x[i] = xq[ps][ks][i];
-      if (p.do_rotary) {
-        float y[16];
-        float cc[16], ss[16];
-        if constexpr (DL != D) {
-          rope_table16_padded<D>(p.cos_cache + (size_t)(L - 1) * HL,
-                                 p.sin_cache + (size_t)(L - 1) * HL, c0, p.interleaved != 0, cc, ss);
-        } else if constexpr (BIG) {
-          float4 lc[4], ls[4];
-          rope_load16<D>(p.cos_cache + (size_t)(L - 1) * HALF, p.sin_cache + (size_t)(L - 1) * HALF,
-                         c0, p.interleaved, lc, ls);
-          rope_pick_all<0>(lc, ls, p.interleaved != 0, cc, ss);
-        } else {
-          rope_pick_all<0>(cq[ks], sq[ks], p.interleaved != 0, cc, ss);
+        for (int i = 0; i < 16; ++i) x[i] = xq[ps][ks][i];
+        if (p.do_rotary) {
+          float y[16];
+          float cc[16], ss[16];
+          if constexpr (DL != D) {
+            rope_table16_padded<D>(p.cos_cache + (size_t)(L - 1) * HL,
+                                   p.sin_cache + (size_t)(L - 1) * HL, c0, p.interleaved != 0, cc, ss);
+          } else if constexpr (BIG) {
+            float4 lc[4], ls[4];
+            rope_load16<D>(p.cos_cache + (size_t)(L - 1) * HALF, p.sin_cache + (size_t)(L - 1) * HALF,
+                           c0, p.interleaved, lc, ls);
+            rope_pick_all<0>(lc, ls, p.interleaved != 0, cc, ss);
+          } else {
+            rope_pick_all<0>(cq[ks], sq[ks], p.interleaved != 0, cc, ss);
+          }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            // split-half partner d +- D/2: up to head_dim 128 the same element
+            // of lane g ^ 2 (32 lanes away; permlane32_swap(a, b) gives [1] =
+            // a of lanes 32-63 on lanes 0-31, [0] = b of lanes 0-31 on lanes
+            // 32-63); at 256 the same lane's chunk ks ^ 2; at the stored width
+            // 192 chunk (ks + 1) % 3 of lane group g + 2 for g < 2 and chunk
+            // (ks + 2) % 3 of lane group g - 2 for g >= 2
+            float half_partner;
+            if constexpr (WIDE) {
+              half_partner = xq[ps][ks ^ 2][i];
+            } else if constexpr (D == 192) {
+              auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(xq[ps][(ks + 1) % 3][i]),
+                                                         __float_as_uint(xq[ps][(ks + 2) % 3][i]),
+                                                         false, false);
+              half_partner = __uint_as_float(g < 2 ? sw[1] : sw[0]);
+            } else {
+              auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[i]),
+                                                         __float_as_uint(x[i]), false, false);
+              half_partner = __uint_as_float(c0 < HALF ? sw[1] : sw[0]);
+            }
+            const float partner = p.interleaved ? x[i ^ 1] : half_partner;
+            const bool first = p.interleaved ? (i & 1) == 0 : c0 < HALF;
+            y[i] = rope_elem(cc[i], ss[i], x[i], partner, first);
+            // padding dims stay 0 whatever the table holds
+            if constexpr (DL != D) y[i] = logical_dim<D>(c0 + i) < 0 ? 0.0f : y[i];
+          }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) x[i] = y[i];
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          // split-half partner d +- D/2: up to head_dim 128 the same element
-          // of lane g ^ 2 (32 lanes away; permlane32_swap(a, b) gives [1] =
-          // a of lanes 32-63 on lanes 0-31, [0] = b of lanes 0-31 on lanes
-          // 32-63); at 256 the same lane's chunk ks ^ 2; at the stored width
-          // 192 chunk (ks + 1) % 3 of lane group g + 2 for g < 2 and chunk
-          // (ks + 2) % 3 of lane group g - 2 for g >= 2
-          float half_partner;
-          if constexpr (WIDE) {
-            half_partner = xq[ps][ks ^ 2][i];
-          } else if constexpr (D == 192) {
-            auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(xq[ps][(ks + 1) % 3][i]),
-                                                       __float_as_uint(xq[ps][(ks + 2) % 3][i]),
-                                                       false, false);
-            half_partner = __uint_as_float(g < 2 ? sw[1] : sw[0]);
-          } else {
-            auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[i]),
-                                                       __float_as_uint(x[i]), false, false);
-            half_partner = __uint_as_float(c0 < HALF ? sw[1] : sw[0]);
-          }
-          const float partner = p.interleaved ? x[i ^ 1] : half_partner;
-          const bool first = p.interleaved ? (i & 1) == 0 : c0 < HALF;
-          y[i] = rope_elem(cc[i], ss[i], x[i], partner, first);
-          // padding dims stay 0 whatever the table holds
-          if constexpr (DL != D) y[i] = logical_dim<D>(c0 + i) < 0 ? 0.0f : y[i];
+          qv[ks][i] = live ? x[i] : 0.0f;
+          amax = fmaxf(amax, fabsf(qv[ks][i]));
+        }
+      }
+      amax = xgroup_max(amax);
+      const float s0 = amax > 0.0f ? amax * (1.0f / 127.0f) : 1.0f;
+      const float inv = 1.0f / s0;
+      const float s1 = s0 * (1.0f / 254.0f);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        int c[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float y = qv[ks][i];
+          const float hi = fminf(fmaxf(rintf(y * inv), -127.0f), 127.0f);
+          const float r1 = y - hi * s0;
+          const float mid = fminf(fmaxf(rintf(r1 * (254.0f * inv)), -127.0f), 127.0f);
+          const float r2 = r1 - mid * s1;
+          const float lo = fminf(fmaxf(rintf(r2 * (64516.0f * inv)), -127.0f), 127.0f);
+          c[i] = live && tq < 3 ? (int)(tq == 0 ? hi : (tq == 1 ? mid : lo)) : 0;
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) x[i] = y[i];
+        for (int w = 0; w < 4; ++w)
+          qB[ps][ks][w] = pack4(c[4 * w], c[4 * w + 1], c[4 * w + 2], c[4 * w + 3]);
       }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        qv[ks][i] = live ? x[i] : 0.0f;
-        amax = fmaxf(amax, fabsf(qv[ks][i]));
-      }
+      // the softmax scale (log2 domain) rides on the term weights
+      const float w0 = s0 * p.scale_log2;
+      qw[ps] = tq == 0 ? w0 : (tq == 1 ? w0 * (1.0f / 254.0f) : (tq == 2 ? w0 * (1.0f / 64516.0f) : 0.0f));
     }
-    amax = xgroup_max(amax);
-    const float s0 = amax > 0.0f ? amax * (1.0f / 127.0f) : 1.0f;
-    const float inv = 1.0f / s0;
-    const float s1 = s0 * (1.0f / 254.0f);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      int c[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float y = qv[ks][i];
-        const float hi = fminf(fmaxf(rintf(y * inv), -127.0f), 127.0f);
-        const float r1 = y - hi * s0;
-        const float mid = fminf(fmaxf(rintf(r1 * (254.0f * inv)), -127.0f), 127.0f);
-        const float r2 = r1 - mid * s1;
-        const float lo = fminf(fmaxf(rintf(r2 * (64516.0f * inv)), -127.0f), 127.0f);
-        c[i] = live && tq < 3 ? (int)(tq == 0 ? hi : (tq == 1 ? mid : lo)) : 0;
-      }
-#pragma unroll
-      for (int w = 0; w < 4; ++w)
-        qB[ps][ks][w] = pack4(c[4 * w], c[4 * w + 1], c[4 * w + 2], c[4 * w + 3]);
-    }
-    // the softmax scale (log2 domain) rides on the term weights
-    const float w0 = s0 * p.scale_log2;
-    qw[ps] = tq == 0 ? w0 : (tq == 1 ? w0 * (1.0f / 254.0f) : (tq == 2 ? w0 * (1.0f / 64516.0f) : 0.0f));
-  }
 
-  // ---- stream the split's tiles, double-buffered --------------------------------
-  // Ping-pong between two tile buffers: the next tile is taken and its load
-  // issued before the current one is computed, so one tile is always in
-  // flight; the loads inside the loop are unconditional once a tile is taken.
-  TileRegs<D> TB;
-  auto tok0 = [&](int tile) { return t_begin + tile * 64 + 16 * g; };
-  auto ld = [&](TileRegs<D>& T, int tile) {
-    load_tile<D>(T, p.pool, sm_pg, tile, p.num_pages, kvh, r, g, n_pages_split);
-  };
-  // the touch loads, consumed (an empty asm use keeps them): issued right
-  // after the first tile, which the loop waits for first anyway
+    // ---- stream the split's tiles, double-buffered --------------------------------
+    // Ping-pong between two tile buffers: the next tile is taken and its load
+    // issued before the current one is computed, so one tile is always in
+    // flight; the loads inside the loop are unconditional once a tile is taken.
+    TileRegs<D> TB;
+    auto tok0 = [&](int tile) { return t_begin + tile * 64 + 16 * g; };
+    auto ld = [&](TileRegs<D>& T, int tile) {
+      load_tile<D>(T, p.pool, sm_pg, tile, p.num_pages, kvh, r, g, n_pages_split);
+    };
+    // the touch loads, consumed (an empty asm use keeps them): issued right
+    // after the first tile, which the loop waits for first anyway
 #pragma unroll
-  for (int j = 0; j < kTouch; ++j) __asm__ volatile("" ::"v"(touch[j]));
-  // (the index for the tile after next is asked for before the next tile's
-  // loads are issued, for the same reason as above)
-  if constexpr (D <= 128) {
-    {
+    for (int j = 0; j < kTouch; ++j) __asm__ volatile("" ::"v"(touch[j]));
+    // (the index for the tile after next is asked for before the next tile's
+    // loads are issued, for the same reason as above)
+    if constexpr (D <= 128) {
       int cur = first;
       for (;;) {
         const int n1 = grab_value(gq);
@@ -618,33 +617,32 @@ __global__ __launch_bounds__(64 * NW, (kInt8OneWavePerSimd<D, G>) ? 1 : 2) void 
         compute_tile<D, G>(TB, st, qB, qw, tok0(n1), k_lo, t_end, r, g, sm_sc[wave]);
         cur = n2;
       }
-    }
-  } else {
-    // head_dim 256: a tile is ~128 registers, so one buffer, refilled by
-    // phase: the next tile's K (and scales) load as soon as this tile's QK is
-    // issued, its V as soon as this tile's PV is (the last tile reloads
-    // itself, so the code stays straight-line)
-    if (have_first) {
-      int cur = first;
-      ld(TA, cur);
-      for (;;) {
-        const int n1 = grab_value(gq);
-        const bool more = n1 < pool_end;
-        const int kn = more ? n1 : cur;
-        // asked for unconditionally (straight-line code); the last one is
-        // never used
-        gq = grab_issue();
-        compute_tile<D, G>(
-            TA, st, qB, qw, tok0(cur), k_lo, t_end, r, g, sm_sc[wave],
-            [&]() { load_tile<D, 1>(TA, p.pool, sm_pg, kn, p.num_pages, kvh, r, g, n_pages_split); },
-            [&]() { load_tile<D, 2>(TA, p.pool, sm_pg, kn, p.num_pages, kvh, r, g, n_pages_split); });
-        if (!more) break;
-        cur = n1;
+    } else {
+      // head_dim 256: a tile is ~128 registers, so one buffer, refilled by
+      // phase: the next tile's K (and scales) load as soon as this tile's QK is
+      // issued, its V as soon as this tile's PV is (the last tile reloads
+      // itself, so the code stays straight-line)
+      if (have_first) {
+        int cur = first;
+        ld(TA, cur);
+        for (;;) {
+          const int n1 = grab_value(gq);
+          const bool more = n1 < pool_end;
+          const int kn = more ? n1 : cur;
+          // asked for unconditionally (straight-line code); the last one is
+          // never used
+          gq = grab_issue();
+          compute_tile<D, G>(
+              TA, st, qB, qw, tok0(cur), k_lo, t_end, r, g, sm_sc[wave],
+              [&]() { load_tile<D, 1>(TA, p.pool, sm_pg, kn, p.num_pages, kvh, r, g, n_pages_split); },
+              [&]() { load_tile<D, 2>(TA, p.pool, sm_pg, kn, p.num_pages, kvh, r, g, n_pages_split); });
+          if (!more) break;
+          cur = n1;
+        }
       }
     }
-  }
 
-  }  // D == 192 || have_first
+  }
 
   // ---- merge the NW waves of the workgroup --------------------------------------
   __shared__ float sm_m[NW][G];

@@ -4,14 +4,16 @@
 //
 // Workgroup = 8 waves = 256 attention rows = (256/G query positions) x (G
 // heads of one kv head), so every K/V tile is loaded once per workgroup and
-// shared by the whole GQA group; each wave owns two 16-row blocks.
+// shared by the whole GQA group; each wave owns two 16-row blocks. (Fewer rows
+// where the waves share out the keys instead, see gqa_prefill_kernel; one row
+// block per wave above head_dim 128.) prefill_plan.h chooses the split.
 // Per 64-token KV tile (4 pages):
 //   staging  the next tile's codes and scales are loaded into registers while
 //            the current tile is computed, then written as f16 into the other
 //            half of a double-buffered LDS tile: K token-major, V in the
 //            permuted k-order of the PV operand; rows padded so the 16-byte
-//            LDS reads are conflict-free. One barrier per tile. int8 codes are
-//            stored exactly (|code| <= 128) and their per-token scales applied
+//            LDS reads are conflict-free. One barrier per tile or two. int8
+//            codes are stored exactly (|code| <= 128) and their per-token scales applied
 //            to the scores and to P; int4 K codes are stored exactly too, V is
 //            dequantised while staged.
 //   S^T      A = K tile (LDS), B = Q^T (registers, f16 of q * scale * log2 e);
@@ -284,7 +286,7 @@ __device__ __forceinline__ void stage_store(const TileStage<D, NT>& S, Tile& T, 
 // loop 137 -> 120 us, the call 178 -> 143 (with the query prologue below).
 //
 // The parameters of a tile are staged one tile ahead of its codes (V's are
-// needed to store them), in a ring of three.
+// needed to store them), in a ring of three (two key groups: of four).
 template <int D>
 struct Int4Params {
   static constexpr int NG = D / 32;
@@ -545,11 +547,11 @@ __device__ __forceinline__ void rope_q_rows(const PrefillParams& p, const int (&
 //
 // KG key groups: the waves form KG groups of NW / KG; every wave stages every
 // tile, but a group computes one tile in KG, so a workgroup holds 1 / KG of
-// the rows and passes them KG tiles at a time. The
-// groups' (m, l, o) meet in LDS at the end. For chunks whose 256-row
-// workgroups would be few (each streaming its keys one tile after the other)
-// or mostly empty; cutting their key range over workgroups instead writes
-// every row's partials to memory and merges them in another launch. KG = 2
+// the rows and passes them KG tiles at a time. The groups' (m, l, o) meet in
+// LDS at the end. For chunks whose 256-row workgroups would be few (each
+// streaming its keys one tile after the other) or mostly empty (prefill_plan);
+// cutting their key range over workgroups instead writes every row's partials
+// to memory and merges them in another launch. KG = 2
 // uses the four tile slots of int8 as one group does; int4 has LDS for a round
 // only, stored behind a second barrier, and so has KG = 4 (int8), which takes
 // one row block per wave (32 rows): the registers of four tiles' loads need
@@ -708,7 +710,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void gqa_prefill_kernel(PrefillPar
   }
   load_stage(t_first);
 
-  // ---- Q^T operand: rows R = wave*32 + rb*16 + r -> (position, head) -------
+  // ---- Q^T operand: rows R = rw * 16 RB + 16 rb + r -> (position, head) ----
   // RoPE(q) * scale * log2(e) as an f16 pair hi + lo (~22 bits: a score's
   // rounding error stays ~2^-20 of its largest term, outlier channels
   // included); lane (r, g) holds dims 32ks + 8g .. +7

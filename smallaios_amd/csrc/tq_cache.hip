@@ -7,9 +7,10 @@
 // (kv_compression.rs:216-268): signs s (the head's xorshift +-1 vector),
 // normalised Walsh-Hadamard butterfly y = H(s*x)/sqrt(D), one min/max
 // quantiser over y (codes of 3, 4 or 8 bits), and, with QJL on (:365-395),
-// the sign bits of r = x - decode(codes) and C = mean|r|. One wave encodes a
-// row, lane l holding dims l + 64 e (D = 64, 128 or 256): every f32 step is the reference's
-// (same operands, same order, no contraction, IEEE division; the running
+// the sign bits of r = x - decode(codes) and C = mean|r|. A wave encodes a row,
+// lane l holding dims l + 64 e (D = 64, 128 or 256), or in passes of several
+// rows D/32 of its lanes do: every f32 result is the reference's (same
+// operands, same order, no contraction, codes of the IEEE quotient; the running
 // sum of |r| is taken in dim order), so codes, scale, zero point, sign bits
 // and C are the reference's bit for bit.
 //
@@ -371,12 +372,12 @@ __global__ __launch_bounds__(64) void tq_write_row_kernel(const TqArgs a, const 
 // lanes once, through LDS, into the words of the position-packed tile (old
 // bits of positions outside the pass kept); one workgroup owns a tile.
 //
-// The work is the serial arithmetic of a row (two butterflies, D IEEE
-// divisions, the D-long sum), not memory. One row per wave at a time ran
-// those chains 64 times over per tile: a 2 x 1024-row pass (8 kv heads, D =
-// 128, 4 bits, QJL, bf16; 23 MB, 3 us at 8 TB/s) took 133 us and takes 14.1 (19
-// with an IEEE division for every code).
-//
+// The work is the serial arithmetic of a row (two butterflies, D quotients,
+// the D-long sum), not memory. One row per wave at a time ran those chains 64
+// times over per tile: a 2 x 1024-row pass (8 kv heads, D = 128, 4 bits, QJL,
+// bf16; 23 MB, 3 us at 8 TB/s) took 133 us and takes 14.1 (19 with an IEEE
+// division for every code instead of the reciprocal).
+
 // A stage across lanes: the partner plus or minus the lane's own value, the
 // sign as an exact product (no select of two sums; the attention kernel's
 // register budget is better off with the select).
